@@ -1188,7 +1188,10 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t hv = lane < nh ? S.hoff[lane] : H;
   const uint32_t hn = lane < nh ? S.hoff[lane + 1u] - hv : 0u;
-  const uint32_t pieces = (hn + kPiece - 1u) / kPiece;
+  // a brick of few atoms is cut finer, so that each of its waves has an item
+  const uint32_t each = (H + (uint32_t)(L::kThreads / 64) - 1u) / (uint32_t)(L::kThreads / 64);
+  const uint32_t piece = each < 4u ? 4u : (each < kPiece ? each : kPiece);
+  const uint32_t pieces = (hn + piece - 1u) / piece;
   const uint32_t pincl = wave_incl_scan_u32(pieces, (int)lane);
   const uint32_t pv = pincl - pieces;  // lanes past the home cells: the item count
   const uint32_t n_items = readlane_u32(pincl, 63);

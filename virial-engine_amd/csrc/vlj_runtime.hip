@@ -32,6 +32,27 @@ constexpr uint32_t kGraphSteps = 16;
 // check before is planned again from its present cell occupancy.
 constexpr double kDefaultFill = 0.9;
 constexpr double kTuneFills[] = {0.8, 0.9, 1.0};
+// A handle of few atoms cuts them into at least this many bricks, of no fewer
+// than kSpreadAtoms home atoms (one wave): with the largest bricks that fit
+// the LDS a small system runs on a handful of the 256 CUs, and a launch lasts
+// as long as one brick (staging 3200 atoms, ~480 home atoms in series per
+// wave). One workgroup per CU is the line: us per step with no spread / 256 /
+// 512 / 1024 bricks: 1000 atoms 35 / 27.5 / 27.5 / 27.5, 50,653 atoms 42 /
+// 38.5 / 45.5 / 57 (past one workgroup per CU the halos staged again cost more than the
+// parallelism gives). Fewer than 64 atoms per brick gains nothing (32: within
+// 2%), 128 keeps half of the small system's gain.
+constexpr double kSpreadBricks = 256.0;
+constexpr double kSpreadAtoms = 64.0;
+// From this many atoms per brick on the LDS limit alone makes enough bricks (a
+// dense brick holds ~460): held to 487, eight slabs of
+// 15,600 atoms ran 1% slower (12% at 244).
+constexpr double kSpreadMost = 384.0;
+constexpr double kNoSpread = 1e300;
+// Atoms per staged cell from which a layer keeps the dense layout however few
+// its bricks stage: a small brick of a liquid fits the sparse layout's 1024
+// atoms, but that layout's build gives each home atom to one lane, which tests
+// a liquid's ~520 candidates one by one.
+constexpr double kSparseCell = 8.0;
 constexpr uint32_t kTuneSteps = 6;
 constexpr uint32_t kTuneMinAtoms = 65536;
 constexpr uint64_t kTuneAutoSteps = 64;
@@ -462,8 +483,10 @@ int capture(vlj_sim* s, uint32_t steps, hipGraphExec_t* out) {
 // from a 2D prefix sum of the three layers' counts over the periodically
 // extended plane. A brick that outgrows LDS later on is cut into parts on
 // the device. A layer whose bricks are held to at most `sparse_fill` of the
-// sparse layout's 1024 atoms takes that layout.
-void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fill, double sparse_fill,
+// sparse layout's 1024 atoms takes that layout. A brick of more than one cell
+// owns at most `spread` atoms, by the larger of the replica's and its staged
+// layers' mean occupancy.
+void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fill, double sparse_fill, double spread,
                    std::vector<uint32_t>& bx, std::vector<uint32_t>& by, std::vector<uint8_t>& bz,
                    std::vector<uint8_t>& sparse) {
   const int nx = (int)R.cells[0], ny = (int)R.cells[1], nz = (int)R.cells[2];
@@ -533,10 +556,12 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
   auto best_shape = [&](int z, int k) {
     Shape b;
     uint32_t best = 0;
+    const double mean_cell = std::max(whole, layers_mean(z, k));
     for (int gy = 1; gy <= std::min(kBrickMax, ny); gy++)
       for (int gx = gy; gx <= std::min(kBrickMax, nx); gx++) {
         const uint32_t home = (uint32_t)(gx * gy * k);
         if (home <= best || home > (uint32_t)kHomeCells || (k + 2) * (gx + 2) * (gy + 2) > kStageCells) continue;
+        if (home > 1u && (double)home * mean_cell > spread) continue;
         const double staged_cells = (double)(k + 2) * (gx + 2) * (gy + 2);
         double windows = 0.0;  // the largest window, with its margin
         const double floor_count = margin((uint64_t)(whole * staged_cells));
@@ -563,8 +588,11 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
   // a brick that stages few atoms takes the sparse layout: few by its own
   // layers' counts, and no more than twice the sparse limit by the
   // replica's mean
-  auto sparse_of = [&](const Shape& b) {
-    return b.fits && b.local <= sparse_limit && b.worst <= 2.0 * sparse_limit ? 1 : 0;
+  auto sparse_of = [&](const Shape& b, int z, int k) {
+    return b.fits && b.local <= sparse_limit && b.worst <= 2.0 * sparse_limit &&
+                   (g_plan.sparse_fill != 0.0 || layers_mean(z, k) < kSparseCell)
+               ? 1
+               : 0;
   };
   bx.assign(nz, 1);
   by.assign(nz, 1);
@@ -575,7 +603,7 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
     one[z] = best_shape(z, 1);
     bx[z] = one[z].gx;
     by[z] = one[z].gy;
-    sparse[z] = (uint8_t)sparse_of(one[z]);
+    sparse[z] = (uint8_t)sparse_of(one[z], z, 1);
   }
   // Layers z, z + 1 (z even) share two-layer bricks when these stage fewer
   // cells per home cell than the two layers' own bricks: a brick stages one
@@ -591,7 +619,7 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
       by[z] = by[z + 1] = two.gy;
       bz[z] = 2;
       bz[z + 1] = 0;
-      sparse[z] = sparse[z + 1] = (uint8_t)sparse_of(two);
+      sparse[z] = sparse[z + 1] = (uint8_t)sparse_of(two, z, 2);
     }
 }
 
@@ -601,6 +629,13 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
 double plan_fill(const vlj_sim* s) { return g_plan.stage_fill != 0.0 ? g_plan.stage_fill : s->fill; }
 double plan_sparse_fill(const vlj_sim* s) {
   return g_plan.sparse_fill != 0.0 ? g_plan.sparse_fill : plan_fill(s);
+}
+
+// Home atoms a brick may own, so that the handle has kSpreadBricks of them.
+double plan_spread(const vlj_sim* s) {
+  if (g_plan.stage_fill != 0.0) return kNoSpread;
+  const double atoms = (double)s->n_total / kSpreadBricks;
+  return atoms > kSpreadMost ? kNoSpread : std::max(kSpreadAtoms, atoms);
 }
 
 // The brick table from the replicas' brick shapes: every replica's dense
@@ -705,8 +740,8 @@ int replan(vlj_sim* s, const std::vector<char>& which, double fill, double* buil
     const Replica& R = s->rep[r];
     std::vector<uint32_t> occ(cn.begin() + R.cell_off, cn.begin() + R.cell_off + R.total_cells);
     HostReplica& H = s->host[r];
-    choose_bricks(R, occ, plan_fill(s) * H.headroom, plan_sparse_fill(s) * H.headroom, H.brick_x, H.brick_y,
-                  H.brick_z, H.sparse);
+    choose_bricks(R, occ, plan_fill(s) * H.headroom, plan_sparse_fill(s) * H.headroom, plan_spread(s), H.brick_x,
+                  H.brick_y, H.brick_z, H.sparse);
   }
   if (g_plan.stage_fill != 0.0) s->fill = saved;
   build_table(s);
@@ -845,7 +880,8 @@ int check_bricks(vlj_sim* s) {
         H.headroom = std::max(0.6, 0.9 * H.headroom);
         std::vector<uint32_t> bx, by;
         std::vector<uint8_t> bz, sp;
-        choose_bricks(rp, occ, plan_fill(s) * H.headroom, plan_sparse_fill(s) * H.headroom, bx, by, bz, sp);
+        choose_bricks(rp, occ, plan_fill(s) * H.headroom, plan_sparse_fill(s) * H.headroom, plan_spread(s), bx, by, bz,
+                      sp);
         which[r] = parts_now || bx != H.brick_x || by != H.brick_y || bz != H.brick_z || sp != H.sparse;
         any = any || which[r];
       }
@@ -920,6 +956,7 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   s->shifted = settings[0].shifted_force != 0;
   uint32_t atom_off = 0, cell_off = 0, scan_off = 0;
   uint64_t list_off = 0, prof_off = 0;
+  s->n_total = (uint32_t)total;
   std::vector<std::vector<uint32_t>> occs(replicas);  // each replica's initial cell occupancy
   for (size_t r = 0; r < replicas; r++) {
     Replica& R = s->rep[r];
@@ -954,7 +991,7 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
     }
     R.atom_block_off = (uint32_t)s->atom_blocks.size();
     R.atom_blocks = (R.count + kBlock - 1) / kBlock;
-    choose_bricks(R, occ, plan_fill(s), plan_sparse_fill(s), s->host[r].brick_x, s->host[r].brick_y,
+    choose_bricks(R, occ, plan_fill(s), plan_sparse_fill(s), plan_spread(s), s->host[r].brick_x, s->host[r].brick_y,
                   s->host[r].brick_z, s->host[r].sparse);
     for (uint32_t b = 0; b < R.count; b += kBlock)
       s->atom_blocks.push_back({(uint32_t)r, atom_off + b, atom_off + std::min(R.count, b + kBlock), 0});
