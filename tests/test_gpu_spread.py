@@ -36,3 +36,58 @@ def test_small_bricks_against_the_oracle(oracle, lj, n, rho, shifted, precision)
         assert list(sim.measure_now().raw) == list(ref.measure().raw)
         np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
         np.testing.assert_array_equal(sim.debug_state()[1], ref.state()[1])
+
+
+@pytest.mark.parametrize("sizes,rho,box,thermostat", [
+    ((8192,), 0.8442, None, 0),              # the one-workgroup rebuild chain's largest system
+    ((8193,), 0.8442, None, 0),              # ... and one atom past it
+    ((1023, 1024, 1025, 1), 0.8442, 10.6, 0),  # around its workgroup's width, and a single atom
+    ((700,), None, 56.1, 0),                 # 8000 cells, most of them empty
+    ((700,), None, 58.9, 0),                 # 9261 cells: past its cell limit
+    ((1025,), 0.8442, None, 1),              # the drift leaves the maxima (Langevin)
+])
+def test_rebuild_chain_against_the_oracle(oracle, lj, sizes, rho, box, thermostat):
+    specs = []
+    for k, n in enumerate(sizes):
+        side = box or (n / rho) ** (1.0 / 3.0)
+        if box and n < 1000:
+            parts = lj.random_insertion_array(n, [side] * 3, 0.9, 1.5, 31 + k)
+        else:
+            parts = lj.lattice_array(n, side, 1.0, 31 + k)
+        th = lj.Langevin(1.0, 1.0, 5 + k) if thermostat else None
+        specs.append((parts, lj.Settings([side] * 3, 2.5, 0.005, skin=0.3, thermostat=th)))
+    sim = lj.Batch(specs)
+    for steps in (1, 17, 62):
+        sim.run(steps)
+    ms, allp = sim.measure_now(), sim.read_particle_array()
+    off = 0
+    for k, (parts, st) in enumerate(specs):
+        ref = oracle.Sim(np.ascontiguousarray(parts["pos"]), np.ascontiguousarray(parts["vel"]), list(st.box_size),
+                         cutoff=2.5, skin=0.3, dt=0.005, thermostat=thermostat, temperature=1.0 if thermostat else 0.0,
+                         friction=1.0 if thermostat else 0.0, seed=5 + k)
+        ref.run(80)
+        r = ref.measure()
+        assert list(ms[k].raw) == list(r.raw) and ms[k].list_rebuilds == r.list_rebuilds, f"replica {k}"
+        pos, vel = ref.read_particles()
+        np.testing.assert_array_equal(allp["pos"][off:off + len(parts)], pos)
+        np.testing.assert_array_equal(allp["vel"][off:off + len(parts)], vel)
+        off += len(parts)
+
+
+def test_forms_change_around_the_decision(oracle, lj):
+    # drift-ahead steps, then a heat exchange (the drift's own maxima), then
+    # drift-ahead steps again: each form's first step decides on its own launch
+    pos, vel = oracle.lattice(1200, 11.3, 1.0, 3)
+    sim = lj.LennardJones((pos, vel), lj.Settings([11.3] * 3, 2.5, 0.004, skin=0.3))
+    ref = oracle.Sim(pos, vel, [11.3] * 3, cutoff=2.5, skin=0.3, dt=0.004)
+    for exchange in (None, lj.HeatExchange((0.0, 2.0), (5.0, 7.0), 0.05), None):
+        sim.set_heat_exchange(exchange)
+        if exchange:
+            ref.set_heat_exchange(exchange.hot, exchange.cold, exchange.energy)
+        else:
+            ref.set_heat_exchange(None, None, 0.0)
+        for steps in (1, 40):
+            sim.run(steps)
+            ref.run(steps)
+            assert list(sim.measure_now().raw) == list(ref.measure().raw)
+            np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])

@@ -165,12 +165,14 @@ struct Buffers {
   double* hexstate;           // per replica: kHexState scales and corrections
   long long* hc;              // heat-current series of replica 0: 3 sums per sample
   double *x, *y, *z, *vx, *vy, *vz, *ax, *ay, *az;           // state, slot order
-  double *x2, *y2, *z2, *vx2, *vy2, *vz2, *ax2, *ay2, *az2;  // reorder target
+  double *x2, *y2, *z2;                                      // the drift-ahead form's next positions
+  double *vx2, *vy2, *vz2, *ax2, *ay2, *az2;                 // v and a in the new order, between build and force
   double *xb, *yb, *zb;                                      // position at last list build
   uint32_t *orig, *orig2;                                    // original index of each slot
-  uint32_t *cell_of, *cell_of2;                              // global cell of each slot
-  uint32_t *unsorted, *sorted;                               // slots in cell order
-  uint32_t *cell_count, *cell_cursor, *cell_scan, *cell_start, *cell_n;
+  uint32_t *cell_of;                                         // global cell of each slot
+  uint32_t *cell_rank;                                       // k_bin to k_scatter: place within the cell's range
+  uint32_t *unsorted, *sorted;                               // old slots in cell order
+  uint32_t *cell_count, *cell_scan, *cell_start, *cell_n;
   uint32_t *bsum, *bprefix;                                  // per scan block
   uint32_t* nbr_count;                                       // list length of each slot
   uint16_t* nbr;                                             // lists of staged indices
@@ -186,14 +188,24 @@ struct Buffers {
   // this step's word (zeroed by the drift, or by the decision of the step
   // before, and counted by the decision) and the next step's
   uint32_t *rebuilding, *rebuilding_next;
-  // Drift-ahead form: kAheadSlots per replica of largest moved^2 since the
-  // list build, taken by the force launch into amax_next (atomicMax) for
-  // the next step, whose k_bin decides from them (bin_decides) in place of
-  // a k_decide launch; each force launch zeroes the set the bin just read.
+  // kAheadSlots per replica of largest moved^2 since the list build
+  // (atomicMax), from which the first kernel of the rebuild chain decides
+  // (bin_decides) in place of a k_decide launch: taken by the drift into amax,
+  // or in the drift-ahead form by the force launch into amax_next for the next
+  // step. Each force launch zeroes the set the decision just read.
   unsigned long long *amax, *amax_next;
   uint32_t bin_decides;
+  uint32_t chain;  // every replica is small enough for k_chain
 };
 constexpr uint32_t kAheadSlots = 64;  // one wave's worth
+
+// k_chain, the rebuild chain of a small replica in one workgroup: its threads,
+// the atoms and cells it takes, and its atoms per thread.
+constexpr uint32_t kChainThreads = 1024;
+constexpr uint32_t kChainAtoms = 8192;
+constexpr uint32_t kChainCells = 8192;
+constexpr uint32_t kChainPer = kChainAtoms / kChainThreads;
+static_assert(kChainAtoms <= 0x10000u && kChainCells <= 0x10000u, "16-bit cells, ranks and places");
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on
 // XCD b % 8). Each table (atom blocks, sort blocks, bricks) is dealt to the

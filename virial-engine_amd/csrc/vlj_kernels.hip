@@ -2,15 +2,15 @@
 //
 // One step is (lennard_jones.rs:1092-1138):
 //   drift       half kick + drift (or BAOAB), displacement since the last
-//               build, one maximum per workgroup (lennard_jones.wgsl:204-276)
-//   decide      per replica: rebuild or not (lennard_jones.wgsl:278-307)
-//   bin         wrap into the box, cell of each atom, count   } rebuild chain,
+//               build (lennard_jones.wgsl:204-276)
+//   bin         rebuild or not (wgsl:278-307); cell, count    } rebuild chain,
 //   scan        exclusive prefix sum of counts                } each kernel
 //   scatter     atoms into their cell's range                 } returns at once
 //   sort        each cell's slots ascending (wave per cell)   } when its replica
-//   reorder     atoms into cell order                         } does not rebuild
-//   build       brick-staged Verlet lists                     } (grid.wgsl, wgsl:419-499)
+//   build       atoms into cell order, wrapped; brick-staged  } does not rebuild
+//               Verlet lists                                  } (grid.wgsl, wgsl:419-499)
 //   force       brick-staged pair forces + second half kick (wgsl:501-574)
+// bin to sort are one kernel, chain, when every replica is small.
 // The sequence is static, so it is captured once into a hipGraph.
 #include <mutex>
 
@@ -131,9 +131,11 @@ __global__ void __launch_bounds__(kBlock) k_decide(Buffers B, int advance) {
 // LANGEVIN: some replica of the launch uses BAOAB (others stay NVE).
 // keep_v: the velocities stay v(t) (the drift-ahead force forms the half
 // step again, as here, before its kick); only the positions move.
+// to_amax: the workgroups' maxima go to the replica's kAheadSlots maxima, from
+// which the rebuild chain's first kernel decides, instead of to bmax (k_decide).
 template <bool LANGEVIN>
-__global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *B.rebuilding = 0u;  // counted again by k_decide
+__global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v, int to_amax) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *B.rebuilding = 0u;  // counted again by the decision
   const uint32_t b = dealt_index(blockIdx.x);
   if (b >= B.n_atom_blocks) return;
   const Range blk = B.atom_blocks[b];
@@ -170,11 +172,9 @@ __global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v) {
     }
     moved = (unsigned long long)__double_as_longlong(dist2(d[0], d[1], d[2]));
   }
-  // One value per workgroup, no atomics (lennard_jones.wgsl:215-220 uses
-  // one global atomicMax per workgroup); k_decide reduces them. (A ticket
-  // per workgroup, so that the replica's last workgroup could decide, is
-  // itself an atomic on one address per replica: from the 4096 workgroups
-  // of a 1M-atom replica it made a step 130 us longer.)
+  // One value per workgroup, into one of 64 maxima (lennard_jones.wgsl:215-220
+  // uses one for all: a single address per replica made the step of a 1M-atom
+  // replica 130 us longer).
   __shared__ unsigned long long wmax[kBlock / 64];
   moved = wave_max_u64(moved);
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = moved;
@@ -183,7 +183,10 @@ __global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v) {
     unsigned long long m = wmax[0];
 #pragma unroll
     for (int w = 1; w < kBlock / 64; w++) m = wmax[w] > m ? wmax[w] : m;
-    B.bmax[b] = m;
+    if (!to_amax)
+      B.bmax[b] = m;
+    else if (m != 0ull)
+      atomicMax(B.amax + (size_t)blk.rep * kAheadSlots + b % kAheadSlots, m);
   }
 }
 
@@ -411,27 +414,39 @@ __device__ __forceinline__ uint32_t run_atomic_add(uint32_t* counter, uint32_t k
   return (uint32_t)__shfl(base, (int)leader, 64) + (lane - leader);
 }
 
-// With bin_decides (drift-ahead steps) every workgroup first takes the rebuild
-// decision of its replica from the maxima the last force launch left (the
-// same rule as k_decide's), and the replica's first atom block records it;
-// such steps come after a k_decide step, so `built` is already set and no
-// workgroup reads a word the recording one writes.
+// R1: the wrapped position, as the rebuild takes it.
+__device__ __forceinline__ uint32_t wrapped_cell(const Replica& R, const Buffers& B, uint32_t i) {
+  return cell_local(R, wrap_one(B.x[i], R.box[0]), wrap_one(B.y[i], R.box[1]), wrap_one(B.z[i], R.box[2]));
+}
+
+// The rebuild decision of replica rep from its kAheadSlots maxima (the same
+// rule as k_decide's), by every workgroup that needs it; the one with `record`
+// set writes it down. Steps that decide here come after a k_decide step, so
+// `built` is already set and no workgroup reads a word the recording one
+// writes.
+__device__ __forceinline__ bool decides(const Buffers& B, uint32_t rep, bool record) {
+  __shared__ unsigned long long moved;
+  if (threadIdx.x < kAheadSlots) {
+    const unsigned long long v = wave_max_u64(B.amax[(size_t)rep * kAheadSlots + threadIdx.x]);
+    if (threadIdx.x == 0) moved = v;
+  }
+  __syncthreads();
+  const double moved2 = __longlong_as_double((long long)moved);
+  const bool rebuild = !B.ctl[rep].built || moved2 > B.rep[rep].half_skin2;
+  if (record && threadIdx.x == 0) decide_from(B, rep, moved2, true);
+  return rebuild;
+}
+
+// The cell of each atom and its place among the cell's atoms (any order), and
+// the cells' counts. With bin_decides every workgroup first takes the rebuild
+// decision of its replica, and the replica's first atom block records it.
 __global__ void __launch_bounds__(kBlock) k_bin(Buffers B) {
   const uint32_t ab = dealt_index(blockIdx.x);
   if (B.bin_decides) {
     if (ab == 0 && threadIdx.x == 0) *B.rebuilding_next = 0u;
     if (ab >= B.n_atom_blocks) return;
     const uint32_t rep = B.atom_blocks[ab].rep;
-    __shared__ unsigned long long moved;
-    if (threadIdx.x < kAheadSlots) {
-      const unsigned long long v = wave_max_u64(B.amax[(size_t)rep * kAheadSlots + threadIdx.x]);
-      if (threadIdx.x == 0) moved = v;
-    }
-    __syncthreads();
-    const double moved2 = __longlong_as_double((long long)moved);
-    const bool rebuild = !B.ctl[rep].built || moved2 > B.rep[rep].half_skin2;
-    if (ab == B.rep[rep].atom_block_off && threadIdx.x == 0) decide_from(B, rep, moved2, true);
-    if (!rebuild) return;
+    if (!decides(B, rep, ab == B.rep[rep].atom_block_off)) return;
   } else {
     if (*B.rebuilding == 0u) return;  // no replica rebuilds this step
     if (ab >= B.n_atom_blocks) return;
@@ -441,17 +456,97 @@ __global__ void __launch_bounds__(kBlock) k_bin(Buffers B) {
   const Replica R = B.rep[blk.rep];
   const uint32_t i = blk.first + threadIdx.x;
   const bool active = i < blk.end;
-  uint32_t c = 0;
+  const uint32_t c = active ? R.cell_off + wrapped_cell(R, B, i) : 0u;
+  const uint32_t rank = run_atomic_add(B.cell_count, c, active);
   if (active) {
-    // R1: positions go back into the box when the lists are rebuilt
-    const double x = wrap_one(B.x[i], R.box[0]), y = wrap_one(B.y[i], R.box[1]), z = wrap_one(B.z[i], R.box[2]);
-    B.x[i] = x;
-    B.y[i] = y;
-    B.z[i] = z;
-    c = R.cell_off + cell_local(R, x, y, z);
     B.cell_of[i] = c;
+    B.cell_rank[i] = rank;
   }
-  run_atomic_add(B.cell_count, c, active);
+}
+
+// The whole chain for replicas of at most kChainAtoms atoms and kChainCells
+// cells, one workgroup each: the decision, the cell counts, their scan, and the
+// atoms in cell order, ascending by old slot in each cell, all in LDS. A launch
+// that only returns costs ~2.1 us, and four of them (and the reorder's, which
+// the build and the force now do) were a third of a small system's step: 1000
+// atoms 28.0 -> 22.6 us. The limit is what one CU sorts faster than the launches
+// over the whole GPU: 8 us at 1000 atoms, 36 us at 15,600 against their ~30
+// (eight slabs of 15,600 atoms: 113 us a step here, 108 with the launches).
+__global__ void __launch_bounds__(kChainThreads) k_chain(Buffers B) {
+  __shared__ uint32_t first[kChainCells + 1];  // counts, then the cell's first place
+  __shared__ uint16_t place[kChainAtoms];      // atoms by place, each cell's in any order
+  __shared__ uint32_t wsum[kChainThreads / 64];
+  const uint32_t r = blockIdx.x, t = threadIdx.x;
+  if (B.bin_decides) {
+    if (r == 0 && t == 0) *B.rebuilding_next = 0u;
+    if (!decides(B, r, true)) return;
+  } else if (!B.ctl[r].rebuild) {
+    return;
+  }
+  const Replica R = B.rep[r];
+  for (uint32_t c = t; c < R.total_cells; c += kChainThreads) first[c] = 0u;
+  __syncthreads();
+  uint32_t own[kChainPer];  // cell | place within the cell << 16
+#pragma unroll
+  for (uint32_t k = 0; k < kChainPer; k++) {
+    own[k] = 0u;
+    if (k * kChainThreads >= R.count) continue;
+    const uint32_t li = k * kChainThreads + t;
+    const bool active = li < R.count;
+    const uint32_t c = active ? wrapped_cell(R, B, R.atom_off + li) : 0u;
+    own[k] = c | run_atomic_add(first, c, active) << 16;
+  }
+  __syncthreads();
+  // exclusive scan of the counts: thread t takes kCells / kThreads cells in a row
+  constexpr uint32_t kPer = kChainCells / kChainThreads;
+  const uint32_t per = (R.total_cells + kChainThreads - 1u) / kChainThreads;
+  uint32_t n[kPer], sum = 0u;
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    const uint32_t c = t * per + k;
+    n[k] = k < per && c < R.total_cells ? first[c] : 0u;
+    sum += n[k];
+  }
+  const uint32_t incl = wave_incl_scan_u32(sum, (int)(t & 63u));
+  if ((t & 63u) == 63u) wsum[t >> 6] = incl;
+  __syncthreads();
+  uint32_t run = incl - sum;
+  for (uint32_t w = 0; w < (t >> 6); w++) run += wsum[w];
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    const uint32_t c = t * per + k;
+    if (k < per && c < R.total_cells) {
+      first[c] = run;
+      B.cell_start[R.cell_off + c] = R.atom_off + run;
+      B.cell_n[R.cell_off + c] = n[k];
+      run += n[k];
+    }
+  }
+  if (t == 0) first[R.total_cells] = R.count;
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kChainPer; k++) {
+    const uint32_t li = k * kChainThreads + t;
+    if (li < R.count) place[first[own[k] & 0xffffu] + (own[k] >> 16)] = (uint16_t)li;
+  }
+  __syncthreads();
+  // an atom's place in its cell is the number of smaller slots in it
+#pragma unroll
+  for (uint32_t k = 0; k < kChainPer; k++) {
+    const uint32_t li = k * kChainThreads + t;
+    if (li < R.count) {
+      const uint32_t c = own[k] & 0xffffu, s0 = first[c], s1 = first[c + 1u];
+      uint32_t at = s0;
+      for (uint32_t m = s0; m < s1; m += 8u) {  // eight reads in flight; past the cell: its last atom again
+        uint32_t p[8];
+#pragma unroll
+        for (uint32_t q = 0; q < 8u; q++) p[q] = place[min(m + q, s1 - 1u)];
+#pragma unroll
+        for (uint32_t q = 0; q < 8u; q++) at += m + q < s1 && p[q] < li ? 1u : 0u;
+      }
+      B.sorted[R.atom_off + at] = R.atom_off + li;
+    }
+  }
 }
 
 // Exclusive scan of counts inside each block of 1024 cells (4 per thread);
@@ -530,9 +625,7 @@ __global__ void __launch_bounds__(kBlock) k_scatter(Buffers B) {
   const Replica R = B.rep[blk.rep];
   const uint32_t i = blk.first + threadIdx.x;
   const bool active = i < blk.end;
-  const uint32_t c = active ? B.cell_of[i] : 0u;
-  const uint32_t rank = run_atomic_add(B.cell_cursor, c, active);
-  if (active) B.unsorted[cell_first_slot(B, R, c) + rank] = i;
+  if (active) B.unsorted[cell_first_slot(B, R, B.cell_of[i]) + B.cell_rank[i]] = i;
 }
 
 // One wave64 per cell: every entry's rank is the number of smaller entries
@@ -561,7 +654,6 @@ __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
     B.cell_start[c] = start;
     B.cell_n[c] = n;
     B.cell_count[c] = 0u;
-    B.cell_cursor[c] = 0u;
     if (n <= kSmallCell) {
       uint32_t e[kSmallCell];
 #pragma unroll
@@ -599,31 +691,6 @@ __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
       }
     }
   }
-}
-
-// Slot t takes the atom at sorted[t] (lennard_jones.wgsl:419-452); the copy
-// goes to the second state set and `build` copies it back.
-__global__ void __launch_bounds__(kBlock) k_reorder(Buffers B) {
-  if (*B.rebuilding == 0u) return;  // no replica rebuilds this step
-  const uint32_t ab = dealt_index(blockIdx.x);
-  if (ab >= B.n_atom_blocks) return;
-  const Range blk = B.atom_blocks[ab];
-  if (!B.ctl[blk.rep].reorder) return;
-  const uint32_t t = blk.first + threadIdx.x;
-  if (t >= blk.end) return;
-  const uint32_t s = B.sorted[t];
-  B.x2[t] = B.x[s];
-  B.y2[t] = B.y[s];
-  B.z2[t] = B.z[s];
-  B.vx2[t] = B.vx[s];
-  B.vy2[t] = B.vy[s];
-  B.vz2[t] = B.vz[s];
-  B.ax2[t] = B.ax[s];
-  B.ay2[t] = B.ay[s];
-  B.az2[t] = B.az[s];
-  B.orig2[t] = B.orig[s];
-  B.cell_of2[t] = B.cell_of[s];
-  B.sorted[t] = t;
 }
 
 // ---------------------------------------------------------------------------
@@ -705,10 +772,11 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 
 // Fills S for brick g from the positions X, Y, Z. Every thread of the
 // workgroup calls it. Returns whether the positions were staged (the
-// neighbourhood holds at most L::kStageMax atoms).
+// neighbourhood holds at most L::kStageMax atoms). `via`, in a rebuild: the
+// positions are still in the old order and not wrapped yet, slot j's at via[j].
 template <class L>
 __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, const double* X, const double* Y,
-                            const double* Z, Stage<L>& S) {
+                            const double* Z, Stage<L>& S, const uint32_t* via = nullptr) {
 #if VLJ_STAGE_PRIO
   __builtin_amdgcn_s_setprio(VLJ_STAGE_PRIO);
 #endif
@@ -807,9 +875,16 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
         const uint32_t c = stage_cell_of(S, e);
         const uint32_t j = S.base[c] + e;
         code[k] = S.image[c];
-        px[k] = X[j];
-        py[k] = Y[j];
-        pz[k] = Z[j];
+        if (via) {
+          const uint32_t s = via[j];
+          px[k] = wrap_one(X[s], R.box[0]);
+          py[k] = wrap_one(Y[s], R.box[1]);
+          pz[k] = wrap_one(Z[s], R.box[2]);
+        } else {
+          px[k] = X[j];
+          py[k] = Y[j];
+          pz[k] = Z[j];
+        }
       }
     }
     if (shifted_any) {
@@ -873,7 +948,7 @@ __device__ __forceinline__ Home home_atom(const Brick& g, const Stage<L>& S, uin
 template <class L>
 __device__ __forceinline__ void staged_pos(const Replica& R, const Stage<L>& S, bool staged, uint32_t e,
                                            const double* X, const double* Y, const double* Z, double& x,
-                                           double& y, double& z) {
+                                           double& y, double& z, const uint32_t* via = nullptr) {
   if (staged) {
     x = S.x[e];
     y = S.y[e];
@@ -883,9 +958,10 @@ __device__ __forceinline__ void staged_pos(const Replica& R, const Stage<L>& S, 
     const uint32_t j = S.base[c] + e;
     double shx, shy, shz;
     image_shift(R, S.image[c], shx, shy, shz);
-    x = X[j] + shx;
-    y = Y[j] + shy;
-    z = Z[j] + shz;
+    const uint32_t s = via ? via[j] : j;
+    x = (via ? wrap_one(X[s], R.box[0]) : X[s]) + shx;
+    y = (via ? wrap_one(Y[s], R.box[1]) : Y[s]) + shy;
+    z = (via ? wrap_one(Z[s], R.box[2]) : Z[s]) + shz;
   }
 }
 
@@ -1086,8 +1162,10 @@ static_assert(kListStride == 64, "entry pos of a list lies (pos / 8) KB + 2 (pos
 // the atom's list length plus its rank in the ballot, and the length grows
 // by the ballot's count. So the entries come out in stencil order dz, dy,
 // dx, then slot (R4), and a sparse cell's 27 neighbours share chunks.
-// On a reorder the workgroup also copies its home atoms' state back from
-// the second set.
+// On a rebuild the atoms are still in the old order (via: the old slot of each
+// new one); the workgroup leaves its home atoms' wrapped positions in xb and
+// their velocities, accelerations and indices in the second set, in the new
+// order, and the force launch that follows takes them from there.
 // Sparse bricks (dilute layers): a lane per home atom, walking its own
 // candidates in list order, the nine runs (dz, dy), each the three staged
 // cells along x, one range of staged atoms. A dilute cell holds a few atoms,
@@ -1096,13 +1174,14 @@ static_assert(kListStride == 64, "entry pos of a list lies (pos / 8) KB + 2 (pos
 // only its own candidates. The lists are the same, entry for entry.
 template <class L>
 __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
-                                            bool staged, const double* X, const double* Y, const double* Z) {
+                                            bool staged, const double* X, const double* Y, const double* Z,
+                                            const uint32_t* via) {
   const uint32_t cap = R.capacity;
   const uint32_t H = S.hoff[home_cells(g)];
   for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
     const Home a = home_atom(g, S, h);
     double xi, yi, zi;
-    staged_pos(R, S, staged, a.e, X, Y, Z, xi, yi, zi);
+    staged_pos(R, S, staged, a.e, X, Y, Z, xi, yi, zi, via);
     const uint32_t li = a.slot - R.atom_off;
     char* lst = (char*)(B.nbr + list_base(R, li));
     uint32_t found = 0u;
@@ -1111,7 +1190,7 @@ __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, 
       const uint32_t s1 = S.off[sc + 3u];
       for (uint32_t q = S.off[sc]; q < s1; q++) {
         double xj, yj, zj;
-        staged_pos(R, S, staged, q, X, Y, Z, xj, yj, zj);
+        staged_pos(R, S, staged, q, X, Y, Z, xj, yj, zj, via);
         const double d2 = dist2(xj - xi, yj - yi, zj - zi);
         if (d2 < R.list_r2 && q != a.e) {
           // byte offset (pos / 8) KB + 2 (pos % 8) = 2 pos + 1008 (pos / 8)
@@ -1138,8 +1217,8 @@ __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, 
 // state is left as it is: the same lists again, for another brick plan.
 template <class L>
 __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
-                                           bool staged, bool moved, bool relist, const double* X, const double* Y,
-                                           const double* Z, uint32_t& next_item) {
+                                           bool staged, bool relist, const double* X, const double* Y,
+                                           const double* Z, const uint32_t* via, uint32_t& next_item) {
   const uint32_t cap = R.capacity;
   const uint32_t total = S.total;
   if (!staged && !relist && threadIdx.x == 0) atomicAdd(&B.ctl[g.rep].stage_global, 1u);
@@ -1149,24 +1228,20 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
     const Home a = home_atom(g, S, h);
     const uint32_t i = a.slot;
     double xi, yi, zi;
-    staged_pos(R, S, staged, a.e, X, Y, Z, xi, yi, zi);
-    if (moved) {  // copy the reordered state back into the main set
-      B.x[i] = xi;
-      B.y[i] = yi;
-      B.z[i] = zi;
-      B.vx[i] = B.vx2[i];
-      B.vy[i] = B.vy2[i];
-      B.vz[i] = B.vz2[i];
-      B.ax[i] = B.ax2[i];
-      B.ay[i] = B.ay2[i];
-      B.az[i] = B.az2[i];
-      B.orig[i] = B.orig2[i];
-      B.cell_of[i] = B.cell_of2[i];
-    }
+    staged_pos(R, S, staged, a.e, X, Y, Z, xi, yi, zi, via);
     if (!relist) {
+      const uint32_t s = via[i];
       B.xb[i] = xi;
       B.yb[i] = yi;
       B.zb[i] = zi;
+      B.vx2[i] = B.vx[s];
+      B.vy2[i] = B.vy[s];
+      B.vz2[i] = B.vz[s];
+      B.ax2[i] = B.ax[s];
+      B.ay2[i] = B.ay[s];
+      B.az2[i] = B.az[s];
+      B.orig2[i] = B.orig[s];
+      B.cell_of[i] = R.cell_off + g.cell0 + (a.hz * R.cells[1] + a.hy) * R.cells[0] + a.hx;
     }
     // A neighbourhood too large for 16-bit staged indices keeps no list;
     // the overflow is reported whatever the capacity, with the staged count
@@ -1178,7 +1253,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
     return;
   }
   if constexpr (L::kSparse) {
-    build_lanes(B, R, S, g, staged, X, Y, Z);
+    build_lanes(B, R, S, g, staged, X, Y, Z, via);
     return;
   }
   // Work items: the atoms of each home cell cut into pieces of at most
@@ -1251,7 +1326,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
           cy[c] = S.y[qs];
           cz[c] = S.z[qs];
         } else if (valid) {
-          staged_pos(R, S, false, q[c], X, Y, Z, cx[c], cy[c], cz[c]);
+          staged_pos(R, S, false, q[c], X, Y, Z, cx[c], cy[c], cz[c], via);
         }
       }
       const uint32_t nc = (T - c0 + 63u) / 64u;  // chunks of this group that hold candidates
@@ -1261,7 +1336,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
       for (uint32_t k = k0; k < k1; k++) {
         const uint32_t e = ebase + k;
         double xi, yi, zi;
-        staged_pos(R, S, staged, e, X, Y, Z, xi, yi, zi);
+        staged_pos(R, S, staged, e, X, Y, Z, xi, yi, zi, via);
         uint32_t f = readlane_u32(found, k - k0);
         char* lst = (char*)(B.nbr + list_base(R, lbase + k));
 #pragma unroll
@@ -1311,7 +1386,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
 // `relist`: every brick of every replica again, from the positions of the
 // last build, after the brick plan changed; nothing else changes.
 template <class L, bool PARTS>
-__global__ void __launch_bounds__(L::kThreads) k_build(Buffers B, int relist) {
+__global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_build(Buffers B, int relist) {
   __shared__ Stage<L> S;
   __shared__ uint32_t next_item;
   if (!relist && *B.rebuilding == 0u) return;  // no replica rebuilds this step
@@ -1321,13 +1396,11 @@ __global__ void __launch_bounds__(L::kThreads) k_build(Buffers B, int relist) {
     const Brick g = B.bricks[gb];
     const Control& ctl = B.ctl[g.rep];
     if (!relist && !ctl.rebuild) return;
-    const bool moved = !relist && ctl.reorder != 0u;
     const Replica R = B.rep[g.rep];
-    const double* X = relist ? B.xb : (moved ? B.x2 : B.x);
-    const double* Y = relist ? B.yb : (moved ? B.y2 : B.y);
-    const double* Z = relist ? B.zb : (moved ? B.z2 : B.z);
+    const double *X = relist ? B.xb : B.x, *Y = relist ? B.yb : B.y, *Z = relist ? B.zb : B.z;
+    const uint32_t* via = relist ? nullptr : B.sorted;
     if (threadIdx.x == 0) next_item = 0u;
-    const bool staged = stage_brick(B, R, g, X, Y, Z, S);  // ends with a barrier
+    const bool staged = stage_brick(B, R, g, X, Y, Z, S, via);  // ends with a barrier
     // A neighbourhood that does not fit is cut into parts when the handle
     // runs the PARTS launches (parts_on), else the brick is built whole from
     // global memory; either way the overflow is counted.
@@ -1344,22 +1417,20 @@ __global__ void __launch_bounds__(L::kThreads) k_build(Buffers B, int relist) {
       if (over && !relist) atomicAdd(&B.ctl[g.rep].stage_overflow, 1u);
     }
     if (cut) return;
-    build_part(B, R, S, g, staged, moved, relist != 0, X, Y, Z, next_item);
+    build_part(B, R, S, g, staged, relist != 0, X, Y, Z, via, next_item);
   } else {
     each_cut_part<L>(B, [&](uint32_t gb, uint32_t code) {
       const Brick brick = B.bricks[gb];
       const Control& ctl = B.ctl[brick.rep];
       if (!relist && !ctl.rebuild) return;
-      const bool moved = !relist && ctl.reorder != 0u;
       const Replica R = B.rep[brick.rep];
-      const double* X = relist ? B.xb : (moved ? B.x2 : B.x);
-      const double* Y = relist ? B.yb : (moved ? B.y2 : B.y);
-      const double* Z = relist ? B.zb : (moved ? B.z2 : B.z);
+      const double *X = relist ? B.xb : B.x, *Y = relist ? B.yb : B.y, *Z = relist ? B.zb : B.z;
+      const uint32_t* via = relist ? nullptr : B.sorted;
       const Brick g = part_brick(brick, code, R);
       __syncthreads();  // the previous part is done with S and next_item
       if (threadIdx.x == 0) next_item = 0u;
-      const bool staged = stage_brick(B, R, g, X, Y, Z, S);
-      build_part(B, R, S, g, staged, moved, relist != 0, X, Y, Z, next_item);
+      const bool staged = stage_brick(B, R, g, X, Y, Z, S, via);
+      build_part(B, R, S, g, staged, relist != 0, X, Y, Z, via, next_item);
     });
   }
 }
@@ -1593,14 +1664,15 @@ __device__ __forceinline__ PairAcc interactions_staged(const Buffers& B, const R
 // entry up to the count, positions through the cell tables.
 template <int PREC, bool SF, bool ENERGIES, class L>
 __device__ __forceinline__ PairAcc interactions_global(const Buffers& B, const Replica& R, const Stage<L>& S,
-                                                    uint32_t i, double xi, double yi, double zi) {
+                                                    const double* X, const double* Y, const double* Z, uint32_t i,
+                                                    double xi, double yi, double zi) {
   const uint32_t cnt = B.nbr_count[i];
   const uint16_t* lst = B.nbr + list_base(R, i - R.atom_off);
   PairAcc a = {0.0, 0.0, 0.0, 0.0, 0.0, 0u, 0u};
   float fx = 0.0f, fy = 0.0f, fz = 0.0f;  // FP32 forces: the current octet's sum
   each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
     double xj, yj, zj;
-    staged_pos(R, S, false, list_index(entry, false), B.x, B.y, B.z, xj, yj, zj);
+    staged_pos(R, S, false, list_index(entry, false), X, Y, Z, xj, yj, zj);
     const double dx = xj - xi, dy = yj - yi, dz = zj - zi;
     if constexpr (PREC == 1 && !ENERGIES) {
       pair_force_f32<SF>(R, dx, dy, dz, dist2(dx, dy, dz), fx, fy, fz);
@@ -1619,9 +1691,10 @@ __device__ __forceinline__ PairAcc interactions_global(const Buffers& B, const R
 
 template <int PREC, bool SF, bool ENERGIES, class L>
 __device__ __forceinline__ PairAcc interactions(const Buffers& B, const Replica& R, const Stage<L>& S, bool staged,
-                                                uint32_t i, double xi, double yi, double zi) {
+                                                const double* X, const double* Y, const double* Z, uint32_t i,
+                                                double xi, double yi, double zi) {
   if (staged) return interactions_staged<PREC, SF, ENERGIES>(B, R, S, i, xi, yi, zi);
-  return interactions_global<PREC, SF, ENERGIES>(B, R, S, i, xi, yi, zi);
+  return interactions_global<PREC, SF, ENERGIES>(B, R, S, X, Y, Z, i, xi, yi, zi);
 }
 
 // New accelerations, one workgroup per brick (gb: its table entry), and
@@ -1634,18 +1707,24 @@ __device__ __forceinline__ PairAcc interactions(const Buffers& B, const Replica&
 // the list build into one of the replica's kAheadSlots maxima of the next
 // step (amax_next), so that step needs no drift launch; the set this step's
 // bin read (amax) is zeroed for the step after.
+// `moved`, when the replica's lists were rebuilt on this step: the state in the
+// new order is where the list build left it (positions in xb, the rest in the
+// second set), and goes to the main set from here.
 template <int PREC, bool SF, class L>
 __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
-                                           uint32_t gb, bool staged, int kick) {
+                                           uint32_t gb, bool staged, int kick, bool moved) {
   const uint32_t H = S.hoff[home_cells(g)];
-  unsigned long long moved = 0ull;
+  const double *X = moved ? B.xb : B.x, *Y = moved ? B.yb : B.y, *Z = moved ? B.zb : B.z;
+  unsigned long long far = 0ull;
   for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
     const Home at = home_atom(g, S, h);
     const uint32_t i = at.slot;
     double xi, yi, zi;
-    staged_pos(R, S, staged, at.e, B.x, B.y, B.z, xi, yi, zi);
+    staged_pos(R, S, staged, at.e, X, Y, Z, xi, yi, zi);
     double* const A[3] = {B.ax, B.ay, B.az};
     double* const V[3] = {B.vx, B.vy, B.vz};
+    const double* const V2[3] = {B.vx2, B.vy2, B.vz2};
+    const double* const A2[3] = {B.ax2, B.ay2, B.az2};
     const double* const XB[3] = {B.xb, B.yb, B.zb};
     // The atom's own v and a, loaded before its pairs so that the loads are
     // in flight while they are summed (the 512-replica batch +3.3%, FCC-1M
@@ -1655,18 +1734,28 @@ __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, c
     double vo[3], ao[3] = {0.0, 0.0, 0.0};
     auto own_state = [&] {
 #pragma unroll
-      for (int k = 0; k < 3; k++) vo[k] = V[k][i];
+      for (int k = 0; k < 3; k++) vo[k] = (moved ? V2[k] : V[k])[i];
       if (kick == 2) {
 #pragma unroll
-        for (int k = 0; k < 3; k++) ao[k] = A[k][i];
+        for (int k = 0; k < 3; k++) ao[k] = (moved ? A2[k] : A[k])[i];
       }
     };
     if constexpr (kEarly) own_state();
-    const PairAcc G = interactions<PREC, SF, false>(B, R, S, staged, i, xi, yi, zi);
+    const PairAcc G = interactions<PREC, SF, false>(B, R, S, staged, X, Y, Z, i, xi, yi, zi);
     if constexpr (!kEarly) own_state();
     const double a[3] = {-24.0 * G.ax, -24.0 * G.ay, -24.0 * G.az};
+    const double xo[3] = {xi, yi, zi};
+    if (moved) {
+      double* const X1[3] = {B.x, B.y, B.z};
+#pragma unroll
+      for (int k = 0; k < 3; k++) X1[k][i] = xo[k];
+      B.orig[i] = B.orig2[i];
+      if (kick == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) V[k][i] = vo[k];
+      }
+    }
     if (kick == 2) {
-      const double* const X[3] = {B.x, B.y, B.z};
       double* const X2[3] = {B.x2, B.y2, B.z2};
       double d[3];
 #pragma unroll
@@ -1675,12 +1764,12 @@ __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, c
         const double v = __builtin_fma(a[k], R.half_dt, half);
         A[k][i] = a[k];
         V[k][i] = v;
-        const double x = __builtin_fma(__builtin_fma(a[k], R.half_dt, v), R.dt, X[k][i]);
+        const double x = __builtin_fma(__builtin_fma(a[k], R.half_dt, v), R.dt, xo[k]);
         X2[k][i] = x;
         d[k] = x - XB[k][i];
       }
       const unsigned long long m = (unsigned long long)__double_as_longlong(dist2(d[0], d[1], d[2]));
-      moved = m > moved ? m : moved;
+      far = m > far ? m : far;
     } else {
 #pragma unroll
       for (int k = 0; k < 3; k++) {
@@ -1690,9 +1779,11 @@ __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, c
     }
   }
   if (kick == 2) {
-    moved = wave_max_u64(moved);
-    if ((threadIdx.x & 63u) == 0 && moved != 0ull)
-      atomicMax(B.amax_next + (size_t)g.rep * kAheadSlots + gb % kAheadSlots, moved);
+    far = wave_max_u64(far);
+    if ((threadIdx.x & 63u) == 0 && far != 0ull)
+      atomicMax(B.amax_next + (size_t)g.rep * kAheadSlots + gb % kAheadSlots, far);
+  }
+  if (kick) {
     if (threadIdx.x == 0)
       for (uint32_t k = gb; k < B.n_replicas * kAheadSlots; k += B.n_bricks) B.amax[k] = 0ull;
   }
@@ -1708,17 +1799,21 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
     if (gb >= layout_end<L>(B)) return;
     const Brick g = B.bricks[gb];
     const Replica R = B.rep[g.rep];
-    const bool staged = stage_brick(B, R, g, B.x, B.y, B.z, S);
+    const bool moved = B.ctl[g.rep].rebuild != 0u;
+    const bool staged =
+        stage_brick(B, R, g, moved ? B.xb : B.x, moved ? B.yb : B.y, moved ? B.zb : B.z, S);
     if (!staged && home_cells(g) > 1u && B.parts_on) return;  // cut into parts
-    force_part<PREC, SF>(B, R, S, g, gb, staged, kick);
+    force_part<PREC, SF>(B, R, S, g, gb, staged, kick, moved);
   } else {
     each_cut_part<L>(B, [&](uint32_t gb, uint32_t code) {
       const Brick brick = B.bricks[gb];
       const Replica R = B.rep[brick.rep];
       const Brick g = part_brick(brick, code, R);
       __syncthreads();  // the previous part is done with S
-      const bool staged = stage_brick(B, R, g, B.x, B.y, B.z, S);
-      force_part<PREC, SF>(B, R, S, g, gb, staged, kick);
+      const bool moved = B.ctl[g.rep].rebuild != 0u;
+      const bool staged =
+          stage_brick(B, R, g, moved ? B.xb : B.x, moved ? B.yb : B.y, moved ? B.zb : B.z, S);
+      force_part<PREC, SF>(B, R, S, g, gb, staged, kick, moved);
     });
   }
 }
@@ -1764,7 +1859,7 @@ __device__ __forceinline__ void measure_part(const Buffers& B, const Replica& R,
       const uint32_t i = at.slot;
       double xi, yi, zi;
       staged_pos(R, S, staged, at.e, B.x, B.y, B.z, xi, yi, zi);
-      const PairAcc a = interactions<PREC, SF, true>(B, R, S, staged, i, xi, yi, zi);
+      const PairAcc a = interactions<PREC, SF, true>(B, R, S, staged, B.x, B.y, B.z, i, xi, yi, zi);
       const double vx = B.vx[i], vy = B.vy[i], vz = B.vz[i];
       const double ke = 0.5 * dist2(vx, vy, vz);
       v[0] = to_fixed(ke, R.energy_fixed);
@@ -2519,13 +2614,14 @@ hipError_t launch_decide(const Buffers& B, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_drift(const Buffers& B, bool langevin, bool keep_v, hipStream_t s) {
+hipError_t launch_drift(const Buffers& B, bool langevin, bool keep_v, bool decide, hipStream_t s) {
   if (!B.n_atom_blocks) return hipSuccess;
+  const dim3 g = grid1(dealt_grid(B.n_atom_blocks));
   if (langevin)
-    hipLaunchKernelGGL(k_drift<true>, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B, keep_v ? 1 : 0);
+    hipLaunchKernelGGL(k_drift<true>, g, dim3(kBlock), 0, s, B, keep_v ? 1 : 0, decide ? 0 : 1);
   else
-    hipLaunchKernelGGL(k_drift<false>, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B, keep_v ? 1 : 0);
-  hipLaunchKernelGGL(k_decide, decide_grid(B), dim3(kBlock), 0, s, B, 1);
+    hipLaunchKernelGGL(k_drift<false>, g, dim3(kBlock), 0, s, B, keep_v ? 1 : 0, decide ? 0 : 1);
+  if (decide) hipLaunchKernelGGL(k_decide, decide_grid(B), dim3(kBlock), 0, s, B, 1);
   return hipGetLastError();
 }
 
@@ -2621,11 +2717,14 @@ static void join_side(hipStream_t s, hipStream_t ss, const Side* side, hipError_
 
 hipError_t launch_rebuild(const Buffers& B, hipStream_t s, const Side* side) {
   if (!B.n_atom_blocks) return hipSuccess;
-  hipLaunchKernelGGL(k_bin, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
-  hipLaunchKernelGGL(k_scan, grid1(B.n_scan_blocks), dim3(kBlock), 0, s, B);
-  hipLaunchKernelGGL(k_scatter, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
-  hipLaunchKernelGGL(k_sort, grid1(dealt_grid(B.n_sort_blocks)), dim3(kBlock), 0, s, B);
-  hipLaunchKernelGGL(k_reorder, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
+  if (B.chain) {
+    hipLaunchKernelGGL(k_chain, dim3(B.n_replicas), dim3(kChainThreads), 0, s, B);
+  } else {
+    hipLaunchKernelGGL(k_bin, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
+    hipLaunchKernelGGL(k_scan, grid1(B.n_scan_blocks), dim3(kBlock), 0, s, B);
+    hipLaunchKernelGGL(k_scatter, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
+    hipLaunchKernelGGL(k_sort, grid1(dealt_grid(B.n_sort_blocks)), dim3(kBlock), 0, s, B);
+  }
   if (!B.n_bricks) return hipGetLastError();
   hipError_t e = hipSuccess;
   const hipStream_t ss = fork_side(B, s, side, e);

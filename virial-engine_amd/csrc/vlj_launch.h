@@ -25,9 +25,12 @@ struct TuneTrial {
 };
 
 hipError_t launch_decide(const Buffers& B, hipStream_t s);
-// The drift and the step's rebuild decision; keep_v: positions only (the
-// drift-ahead form's first step).
-hipError_t launch_drift(const Buffers& B, bool langevin, bool keep_v, hipStream_t s);
+// The drift; keep_v: positions only (the drift-ahead form's first step).
+// decide: the step's rebuild decision on its own launch, which also clears the
+// maxima that later steps decide from (needed first after a change of form);
+// without it the drift leaves its maxima in B.amax for launch_rebuild to
+// decide from (B.bin_decides).
+hipError_t launch_drift(const Buffers& B, bool langevin, bool keep_v, bool decide, hipStream_t s);
 hipError_t launch_rebuild(const Buffers& B, hipStream_t s, const Side* side = nullptr);
 // The lists of every replica again from the positions of the last build
 // (xb), for a new brick table; the cut marks of the table must start at

@@ -124,6 +124,9 @@ struct vlj_sim {
   // positions of the present state. `orient`: whether the sets are swapped
   // from their allocation.
   bool ahead = false;
+  // The other forms: B.amax is clear for the drift's maxima (the last step was
+  // no drift-ahead one).
+  bool maxima_clear = false;
   int orient = 0;
   bool primed = false;
   uint64_t steps = 0;
@@ -403,6 +406,12 @@ int check_device(vlj_sim* s) {
 // thermostat or heat exchange acts between the half steps).
 bool drift_ahead(const vlj_sim* s) { return !s->any_langevin && !s->any_nose_hoover && !s->any_heat_exchange; }
 
+// Whether the next step has the form of the one before it: the drift-ahead
+// form with drifted positions at hand, or the other with clear maxima. The
+// first step after a change of form takes the rebuild decision on its own
+// launch, and only the steps after it are captured.
+bool settled(const vlj_sim* s) { return drift_ahead(s) ? s->ahead : s->maxima_clear; }
+
 // Swaps the two position sets and the two rebuild words.
 void flip_positions(vlj_sim* s) {
   Buffers& B = s->B;
@@ -419,17 +428,17 @@ int enqueue_step(vlj_sim* s, hipEvent_t* around_force = nullptr) {
   if (s->any_nose_hoover) HIP_TRY(s, launch_nh_half(s->B, false, s->stream));
   if (fused && s->ahead) {
     flip_positions(s);  // the positions the last force launch drifted
-    Buffers B = s->B;
-    B.bin_decides = 1u;  // the rebuild decision in k_bin, from the force launch's maxima
-    HIP_TRY(s, launch_rebuild(B, s->stream, &s->side));
   } else {
-    HIP_TRY(s, launch_drift(s->B, s->any_langevin, fused, s->stream));
-    HIP_TRY(s, launch_rebuild(s->B, s->stream, &s->side));
+    HIP_TRY(s, launch_drift(s->B, s->any_langevin, fused, !settled(s), s->stream));
   }
+  Buffers B = s->B;
+  B.bin_decides = settled(s) ? 1u : 0u;  // from the maxima of the last force launch, or of the drift
+  HIP_TRY(s, launch_rebuild(B, s->stream, &s->side));
   if (around_force) HIP_TRY(s, hipEventRecord(around_force[0], s->stream));
   HIP_TRY(s, launch_force(s->B, s->precision, s->shifted, fused ? 2 : 1, s->stream, &s->side));
   if (around_force) HIP_TRY(s, hipEventRecord(around_force[1], s->stream));
   s->ahead = fused;
+  s->maxima_clear = !fused;
   if (s->any_nose_hoover) HIP_TRY(s, launch_nh_half(s->B, true, s->stream));
   if (s->any_heat_exchange) HIP_TRY(s, launch_heat_exchange(s->B, s->stream));
   return VLJ_OK;
@@ -451,13 +460,14 @@ void drop_graphs(vlj_sim* s) {
 int capture(vlj_sim* s, uint32_t steps, hipGraphExec_t* out) {
   hipGraph_t g = nullptr;
   const Buffers saved = s->B;
-  const bool ahead = s->ahead;
+  const bool ahead = s->ahead, maxima_clear = s->maxima_clear;
   const int orient = s->orient;
   HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
   int rc = VLJ_OK;
   for (uint32_t t = 0; t < steps && rc == VLJ_OK; t++) rc = enqueue_step(s);
   s->B = saved;
   s->ahead = ahead;
+  s->maxima_clear = maxima_clear;
   s->orient = orient;
   hipError_t e = hipStreamEndCapture(s->stream, &g);
   if (rc != VLJ_OK) {
@@ -1065,9 +1075,9 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
                   &B.x2, &B.y2, &B.z2, &B.vx2, &B.vy2, &B.vz2, &B.ax2, &B.ay2, &B.az2,
                   &B.xb, &B.yb, &B.zb};
   for (double** p : d) A(p, N);
-  uint32_t** u[] = {&B.orig, &B.orig2, &B.cell_of, &B.cell_of2, &B.unsorted, &B.sorted, &B.nbr_count};
+  uint32_t** u[] = {&B.orig, &B.orig2, &B.cell_of, &B.cell_rank, &B.unsorted, &B.sorted, &B.nbr_count};
   for (uint32_t** p : u) A(p, N);
-  uint32_t** c[] = {&B.cell_count, &B.cell_cursor, &B.cell_scan, &B.cell_start, &B.cell_n};
+  uint32_t** c[] = {&B.cell_count, &B.cell_scan, &B.cell_start, &B.cell_n};
   for (uint32_t** p : c) A(p, C);
   A(&B.bsum, s->scan_blocks.size());
   A(&B.bprefix, s->scan_blocks.size());
@@ -1095,6 +1105,9 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   B.n_scan_blocks = (uint32_t)s->scan_blocks.size();
   B.n_sort_blocks = (uint32_t)s->sort_blocks.size();
   B.n_replicas = (uint32_t)replicas;
+  B.chain = std::all_of(s->rep.begin(), s->rep.end(), [](const Replica& R) {
+    return R.count <= vlj::kChainAtoms && R.total_cells <= vlj::kChainCells;
+  });
 
   // Host-side initial state: wrapped positions, slot = original index.
   std::vector<double> h(N);
@@ -1127,9 +1140,8 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   B.amax_next = B.amax + replicas * kAheadSlots;
   if (e == hipSuccess) e = hipMemset(B.cut, 0, std::max<size_t>(s->bricks.size(), 1) * 4);
   if (e == hipSuccess) e = hipMemset(B.cut_groups, 0, std::max<size_t>((s->bricks.size() + kCutGroup - 1) / kCutGroup, 1) * 4);
-  // Zeroed once here; afterwards the sort kernel leaves them zero.
+  // Zeroed once here; afterwards the sort kernel leaves it zero.
   if (e == hipSuccess) e = hipMemset(B.cell_count, 0, std::max<size_t>(C, 1) * 4);
-  if (e == hipSuccess) e = hipMemset(B.cell_cursor, 0, std::max<size_t>(C, 1) * 4);
   if (e == hipSuccess) e = hipMemset(B.tickets, 0, 16);
   if (e == hipSuccess) e = hipMemset(B.flags, 0, 12);
   B.rebuilding = B.flags;
@@ -1181,9 +1193,8 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
   rc = check_bricks(s);
   if (rc != VLJ_OK) return rc;
   uint64_t left = steps;
-  // The captured drift-ahead steps start from drifted positions: the first
-  // step after a change of form drifts on its own launch.
-  if (drift_ahead(s) && !s->ahead && left > 0) {
+  // The captured steps start from a step of their own form.
+  if (!settled(s) && left > 0) {
     rc = enqueue_step(s);
     if (rc != VLJ_OK) return rc;
     left--;
@@ -1203,7 +1214,10 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
   }
   // what the replayed steps leave: drifted positions in B.x2 after
   // drift-ahead steps, none after the others (which use B.x2 as scratch)
-  if (steps > 0) s->ahead = drift_ahead(s);
+  if (steps > 0) {
+    s->ahead = drift_ahead(s);
+    s->maxima_clear = !s->ahead;
+  }
   s->steps += steps;
   return check_bricks(s);
 }
@@ -1732,8 +1746,8 @@ int vlj_debug_cells(vlj_sim* sim, uint32_t* cell_of, uint32_t* cell_start, uint3
     cell_start[R.total_cells] = R.count;
   }
   if (sorted && rc == VLJ_OK) {
-    rc = read_dev(sim, sorted, B.sorted + R.atom_off, (size_t)R.count * 4);
-    for (uint32_t i = 0; i < R.count && rc == VLJ_OK; i++) sorted[i] -= R.atom_off;
+    // every rebuild leaves the atoms in cell order (R8)
+    for (uint32_t i = 0; i < R.count; i++) sorted[i] = i;
   }
   return rc;
 }
@@ -1752,12 +1766,11 @@ int vlj_debug_lists(vlj_sim* sim, uint32_t* counts, uint32_t* entries) {
     // staging order from the cell tables to turn them into slots.
     const size_t padded = (size_t)((R.count + kListStride - 1) / kListStride) * kListStride;
     std::vector<uint16_t> t((size_t)list_octets(R.capacity) * 8u * padded);
-    std::vector<uint32_t> cell_of(R.count), start(R.total_cells), ncell(R.total_cells), sorted(R.count);
+    std::vector<uint32_t> cell_of(R.count), start(R.total_cells), ncell(R.total_cells);
     rc = read_dev(sim, t.data(), B.nbr + R.list_off, t.size() * 2);
     if (rc == VLJ_OK) rc = read_dev(sim, cell_of.data(), B.cell_of + R.atom_off, (size_t)R.count * 4);
     if (rc == VLJ_OK) rc = read_dev(sim, start.data(), B.cell_start + R.cell_off, (size_t)R.total_cells * 4);
     if (rc == VLJ_OK) rc = read_dev(sim, ncell.data(), B.cell_n + R.cell_off, (size_t)R.total_cells * 4);
-    if (rc == VLJ_OK) rc = read_dev(sim, sorted.data(), B.sorted + R.atom_off, (size_t)R.count * 4);
     if (rc != VLJ_OK) return rc;
     const int nx = (int)R.cells[0], ny = (int)R.cells[1], nz = (int)R.cells[2];
     for (uint32_t i = 0; i < R.count; i++) {
@@ -1788,7 +1801,7 @@ int vlj_debug_lists(vlj_sim* sim, uint32_t* counts, uint32_t* entries) {
           const uint32_t e = list_index(t[base + list_entry(k)], staged);
           size_t sc = std::upper_bound(off.begin(), off.end(), e) - off.begin() - 1;
           while (sc + 1 < off.size() && off[sc + 1] <= e) sc++;
-          slot = sorted[first[sc] + (e - off[sc])] - R.atom_off;
+          slot = first[sc] + (e - off[sc]);
         }
         entries[(size_t)i * R.capacity + k] = slot;
       }
