@@ -319,8 +319,8 @@ int vlj_fixed_sum(const double *values, size_t count, double fixed_scale, int64_
  * are device pointers the caller owns, `stream` is a hipStream_t (NULL: the
  * default stream), and the call only enqueues: *out is written when the
  * stream gets there. It allocates nothing: its partial sums (one per
- * workgroup, at most 1024) and a ticket live in a device array of about
- * 8.5 KB inside the library, one copy per GPU, held until the process ends.
+ * workgroup, at most 256) and a ticket live in a device array of about
+ * 2.3 KB inside the library, one copy per GPU, held until the process ends.
  * At most 2^36 values (VLJ_E_INVALID beyond). Calls that overlap on one GPU
  * (from other threads or streams) race on that array. */
 int vlj_fixed_sum_device(const double *values, size_t count, double fixed_scale, int64_t *out,
