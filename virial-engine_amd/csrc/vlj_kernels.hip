@@ -1460,6 +1460,20 @@ __device__ __forceinline__ double rcp_rn(double x) {
   return __builtin_fma(e, y, y);
 }
 
+// n / x correctly rounded, for x as in rcp_rn and a quotient that is a normal
+// number or zero: rcp_estimate(x) is the estimate after its two Newton-Raphson
+// steps, from which any number of quotients by x take one residual correction
+// each, as the IEEE division sequence does (rcp_rn is the one of n = 1).
+__device__ __forceinline__ double rcp_estimate(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+}
+__device__ __forceinline__ double div_rn(double n, double x, double y) {
+  const double q = n * y;
+  return __builtin_fma(__builtin_fma(-x, q, n), y, q);
+}
+
 // 1 / q correctly rounded in FP32, for a positive normal q whose reciprocal
 // is normal (R5f's 1.0f / q): the hardware estimate (within one ulp), one
 // Newton-Raphson correction y + y (1 - q y) with both steps fused (1 - q y
@@ -1599,6 +1613,30 @@ __device__ __forceinline__ void each_entry(const uint16_t* lst, uint32_t cnt, F&
       const uint32_t k = 8u * o + c;
       if (k < cnt) f(k, (w[c >> 1] >> ((c & 1u) * 16u)) & 0xffffu);
     }
+    cur = nxt;
+  }
+}
+
+// f(x, y, z) for each whole octet of a list of cnt entries in order, with the
+// staged positions of its eight entries (pads give the far sentinel); the next
+// octet's load is in flight while this one is taken.
+template <class L, class F>
+__device__ __forceinline__ void each_octet(const Stage<L>& S, const uint16_t* lst, uint32_t cnt, F&& f) {
+  const uint32_t no = (cnt + 7u) / 8u;
+  const uint32_t last = no > 0u ? no - 1u : 0u;
+  u32x4 cur = load_octet(lst, 0u, last);
+  for (uint32_t o = 0; o < no; o++) {
+    const u32x4 nxt = load_octet(lst, o + 1u, last);
+    const uint32_t w[4] = {cur.x, cur.y, cur.z, cur.w};
+    double x[8], y[8], z[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const uint32_t off = (w[c >> 1] >> ((c & 1) * 16)) & 0xffffu;  // 8 e
+      x[c] = *(const double*)((const char*)S.x + off);
+      y[c] = *(const double*)((const char*)S.y + off);
+      z[c] = *(const double*)((const char*)S.z + off);
+    }
+    f(x, y, z);
     cur = nxt;
   }
 }
@@ -2401,6 +2439,37 @@ __global__ void __launch_bounds__(L::kThreads, WIDE && !PARTS && !L::kSparse ? 4
 // sample `sample` of the series. Pair terms in FP64.
 // ---------------------------------------------------------------------------
 
+// One pair's terms: half its energy into e, (F . v) r / r^2 d into pr. A pair
+// outside the cutoff adds zeros.
+template <bool SF>
+__device__ __forceinline__ void heat_pair(const Replica& R, double dx, double dy, double dz, const double v[3],
+                                          double& e, double pr[3]) {
+  const double r2 = dist2(dx, dy, dz);
+  const bool hit = r2 < R.rc2;
+  const double y = rcp_estimate(r2);
+  const double inv2 = div_rn(1.0, r2, y);
+  const double s6 = inv2 * inv2 * inv2;
+  double rf = s6 * __builtin_fma(48.0, s6, -24.0);
+  const double t = 4.0 * s6;
+  double u = __builtin_fma(t, s6, -t) - R.shift;
+  if (SF) {
+    const double r = __builtin_sqrt(r2);
+    rf = __builtin_fma(-r, R.force_shift, rf);
+    u = __builtin_fma(r - R.rc, R.force_shift, u);
+  }
+  e += hit ? 0.5 * u : 0.0;
+  const double dv = __builtin_fma(dz, v[2], __builtin_fma(dy, v[1], dx * v[0]));
+  const double q = hit ? div_rn(dv * rf, r2, y) : 0.0;
+  pr[0] = __builtin_fma(dx, q, pr[0]);
+  pr[1] = __builtin_fma(dy, q, pr[1]);
+  pr[2] = __builtin_fma(dz, q, pr[2]);
+}
+
+// From LDS the list is taken in whole octets (pads meet the far sentinel), as
+// the force takes it: the eight gathers of each coordinate are in flight
+// together and the pairs carry no branch, and both quotients by r^2 share one
+// reciprocal: 18.7 us for a sample of 3458 atoms, against ~26 entry by entry with
+// two IEEE divisions (37 on the larger bricks it had then).
 template <bool SF, class L>
 __device__ __forceinline__ void heat_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
                                           bool staged, long long jsum[kSlots]) {
@@ -2415,28 +2484,18 @@ __device__ __forceinline__ void heat_part(const Buffers& B, const Replica& R, co
     double pr[3] = {0.0, 0.0, 0.0};
     const uint32_t cnt = B.nbr_count[i];
     const uint16_t* lst = B.nbr + list_base(R, i - R.atom_off);
-    each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
-      double xj, yj, zj;
-      staged_pos(R, S, staged, list_index(entry, staged), B.x, B.y, B.z, xj, yj, zj);
-      const double d[3] = {xj - xi, yj - yi, zj - zi};
-      const double r2 = dist2(d[0], d[1], d[2]);
-      if (!(r2 < R.rc2)) return;
-      const double inv2 = 1.0 / r2;
-      const double s6 = inv2 * inv2 * inv2;
-      double rf = s6 * __builtin_fma(48.0, s6, -24.0);
-      const double t = 4.0 * s6;
-      double u = __builtin_fma(t, s6, -t) - R.shift;
-      if (SF) {
-        const double r = __builtin_sqrt(r2);
-        rf = __builtin_fma(-r, R.force_shift, rf);
-        u = __builtin_fma(r - R.rc, R.force_shift, u);
-      }
-      e += 0.5 * u;
-      const double dv = __builtin_fma(d[2], v[2], __builtin_fma(d[1], v[1], d[0] * v[0]));
-      const double q = dv * rf / r2;
+    if (staged) {
+      each_octet(S, lst, cnt, [&](const double x[8], const double y[8], const double z[8]) {
 #pragma unroll
-      for (int a = 0; a < 3; a++) pr[a] = __builtin_fma(d[a], q, pr[a]);
-    });
+        for (int c = 0; c < 8; c++) heat_pair<SF>(R, x[c] - xi, y[c] - yi, z[c] - zi, v, e, pr);
+      });
+    } else {
+      each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
+        double xj, yj, zj;
+        staged_pos(R, S, false, list_index(entry, false), B.x, B.y, B.z, xj, yj, zj);
+        heat_pair<SF>(R, xj - xi, yj - yi, zj - zi, v, e, pr);
+      });
+    }
 #pragma unroll
     for (int a = 0; a < 3; a++) jsum[a] += to_fixed(__builtin_fma(e, v[a], 0.5 * pr[a]), 4294967296.0);
   }
@@ -2492,6 +2551,15 @@ __device__ __forceinline__ void render_part(const Buffers& B, const Replica& R, 
     double v2 = 0.0;
     const uint32_t cnt = B.nbr_count[i];
     const uint16_t* lst = B.nbr + list_base(R, i - R.atom_off);
+    if (staged && R.drawn != 1u) {
+      each_octet(S, lst, cnt, [&](const double x[8], const double y[8], const double z[8]) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+          const double r2 = dist2(x[c] - xi, y[c] - yi, z[c] - zi);
+          near += r2 < R.rc2 && r2 < kNearR2 ? 1u : 0u;
+        }
+      });
+    } else
     each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
       const uint32_t e = list_index(entry, staged);
       double xj, yj, zj;
