@@ -147,3 +147,21 @@ def test_fp32_forces_profile_adds_up(oracle, lj):
     assert slabs[:, 1:4].sum() == pytest.approx(2.0 * m.kinetic, rel=1e-9)
     assert slabs[:, 7].sum() == pytest.approx(m.potential, rel=1e-5)
     assert (raw[20 * 8:] / TWO32).sum() == pytest.approx(m.virial, rel=1e-5)
+
+
+@pytest.mark.parametrize("bins", [37, 256, 257])
+def test_profile_of_pairs_beyond_the_fast_conversion(oracle, lj, bins):
+    # pairs 0.3 apart along z: virial shares of up to ~1e7, past the range the
+    # short conversion to fixed point takes (2^18), over slabs a tenth of the pair
+    # and wider, summed in LDS (up to 256 slabs) and straight into the profile
+    pos, vel = oracle.lattice(216, 12.0, 1.0, 3)
+    pos = np.concatenate([pos, pos[::18] + [0.0, 0.05, 0.3]])
+    vel = np.concatenate([vel, vel[::18]])
+    sim = lj.LennardJones((pos, vel), lj.Settings([12.0] * 3, 2.5, 0.001, skin=0.3, profile_bins=bins))
+    ref = oracle.Sim(pos, vel, [12.0] * 3, dt=0.001)
+    ref.set_profile_bins(bins)
+    sim.sample_profile()
+    ref.sample_profile()
+    raw = sim.read_profile_raw()[0]
+    assert np.abs(raw).max() > 2 ** 51
+    np.testing.assert_array_equal(raw, ref.read_profile()[0])

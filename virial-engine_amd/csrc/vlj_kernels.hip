@@ -1959,18 +1959,55 @@ __global__ void __launch_bounds__(L::kThreads) k_measure(Buffers B) {
 constexpr uint32_t kProfileLdsBins = 256;
 constexpr double kProfileOne = 4294967296.0;  // fixed point: 2^32 per unit
 
+// to_fixed(x, 2^32) for |x| below kMagicMost: x 2^32 added to 1.5 2^52 rounds to
+// an integer, ties to even, in the sum's last bits (three instructions for nine).
+constexpr double kMagic = 6755399441055744.0;
+constexpr double kMagicMost = 262144.0;  // 2^18: x 2^32 below 2^50
+__device__ __forceinline__ long long to_profile_small(double x) {
+  return __double_as_longlong(__builtin_fma(x, kProfileOne, kMagic)) - __double_as_longlong(kMagic);
+}
+
+// LDS of a workgroup that sums its brick's profile before adding it to the
+// replica's: per slab the virial's three sums, in kCopies copies that lanes take
+// in turn (a wave's 64 segments cross the same few slabs, and 64-bit LDS adds to
+// one address go one after the other; copies of a slab lie in banks of their
+// own), and the five per-atom sums.
+template <class L>
+struct ProfileBins {
+  static constexpr uint32_t kCopies = L::kSparse ? 2u : 8u;
+  long long w[3][kProfileLdsBins * kCopies];
+  long long atom[5][kProfileLdsBins];  // count, v_x^2, v_y^2, v_z^2, potential
+  long long total[3];                  // the whole-box W_aa
+};
+
+// Where a sum goes: the workgroup's LDS (LDS), or straight into the replica's
+// profile. A template, so that the adds are LDS instructions: chosen at run time
+// the compiler merged the two into flat atomics, which took 3 times as long.
+template <class L, bool LDS>
 struct ProfileSink {
-  long long* lds;
+  ProfileBins<L>* lds;
   long long* global;
-  bool use_lds;
-  __device__ __forceinline__ void add(uint32_t k, long long v) const {
-    if (v == 0) return;
-    if (use_lds)
-      atomicAdd((unsigned long long*)(lds + k), (unsigned long long)v);
-    else
-      atomicAdd((unsigned long long*)(global + k), (unsigned long long)v);
+  __device__ __forceinline__ void virial(uint32_t b, uint32_t a, long long v) const {
+    if constexpr (LDS)
+      atomicAdd((unsigned long long*)&lds->w[a][b * ProfileBins<L>::kCopies + threadIdx.x % ProfileBins<L>::kCopies],
+                (unsigned long long)v);
+    else if (v != 0)
+      atomicAdd((unsigned long long*)(global + b * kProfileSums + 4u + a), (unsigned long long)v);
   }
-  __device__ __forceinline__ void add(uint32_t k, double x) const { add(k, to_fixed(x, kProfileOne)); }
+  // sum q of slab b: the count, v_a^2 or the potential
+  __device__ __forceinline__ void atom(uint32_t b, uint32_t q, long long v) const {
+    if constexpr (LDS)
+      atomicAdd((unsigned long long*)&lds->atom[q == 7u ? 4u : q][b], (unsigned long long)v);
+    else if (v != 0)
+      atomicAdd((unsigned long long*)(global + b * kProfileSums + q), (unsigned long long)v);
+  }
+  // a pair's virial share to slab b; SMALL: every |w_a| is below kMagicMost
+  template <bool SMALL>
+  __device__ __forceinline__ void add_virial(uint32_t b, const double w[3], double share) const {
+#pragma unroll
+    for (uint32_t a = 0; a < 3u; a++)
+      virial(b, a, SMALL ? to_profile_small(w[a] * share) : to_fixed(w[a] * share, kProfileOne));
+  }
 };
 
 // The virial shares of one atom's pairs to the slab below its own slab,
@@ -1986,111 +2023,16 @@ struct SlabWindow {
 #pragma unroll
       for (int a = 0; a < 3; a++) w[k][a] = 0.0;
   }
-  // w_a share to slab b (unwrapped), k = b - hb from the atom's (-1, 0, 1
-  // fit). Each sum takes fma(f, 1, sum) = sum + f or fma(f, 0, sum) = sum:
-  // one instruction per sum and no select (a non-finite share, from atoms
-  // on top of each other, spoils all three of the atom's sums instead of
-  // one).
-  __device__ __forceinline__ void add(int k, int b, int bins, const double wv[3], double share,
-                                      const ProfileSink& sink) {
-    if (k >= -1 && k <= 1) {
+  // the pair's shares dn, own and up to the three slabs (0 for one it does not touch)
+  __device__ __forceinline__ void add(const double wv[3], double dn, double own, double up) {
 #pragma unroll
-      for (int kk = 0; kk < 3; kk++) {
-        const double sel = kk == k + 1 ? 1.0 : 0.0;
-#pragma unroll
-        for (int a = 0; a < 3; a++) w[kk][a] = __builtin_fma(wv[a] * share, sel, w[kk][a]);
-      }
-    } else {
-      const uint32_t slab = (uint32_t)(((b % bins) + bins) % bins);
-#pragma unroll
-      for (int a = 0; a < 3; a++) sink.add(slab * kProfileSums + 4u + (uint32_t)a, wv[a] * share);
+    for (int a = 0; a < 3; a++) {
+      w[0][a] += wv[a] * dn;
+      w[1][a] += wv[a] * own;
+      w[2][a] += wv[a] * up;
     }
   }
 };
-
-template <bool SF, class L>
-__device__ __forceinline__ void profile_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
-                                             bool staged, const ProfileSink& sink, long long whole[3]) {
-  const uint32_t bins = R.prof_bins;
-  const double width = R.bin_width;
-  const double iw = 1.0 / width;  // slab of z: floor(z iw)
-  const int ibins = (int)bins;
-  const uint32_t H = S.hoff[home_cells(g)];
-  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
-    const Home at = home_atom(g, S, h);
-    const uint32_t i = at.slot;
-    double xi, yi, zi;
-    staged_pos(R, S, staged, at.e, B.x, B.y, B.z, xi, yi, zi);
-    const double zw = wrap_one(zi, R.box[2]);
-    const int hb = (int)floor(zw * iw);  // the slab the shares are counted from
-    const uint32_t home = (uint32_t)(hb < 0 ? 0 : (hb > ibins - 1 ? ibins - 1 : hb));
-    sink.add(home * kProfileSums, 1.0);
-    const double v[3] = {B.vx[i], B.vy[i], B.vz[i]};
-#pragma unroll
-    for (int a = 0; a < 3; a++) sink.add(home * kProfileSums + 1u + (uint32_t)a, v[a] * v[a]);
-    double pe = 0.0, total[3] = {0.0, 0.0, 0.0};
-    SlabWindow win;
-    win.clear();
-    const uint32_t cnt = B.nbr_count[i];
-    const uint16_t* lst = B.nbr + list_base(R, i - R.atom_off);
-    each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
-      double xj, yj, zj;
-      staged_pos(R, S, staged, list_index(entry, staged), B.x, B.y, B.z, xj, yj, zj);
-      const double d[3] = {xj - xi, yj - yi, zj - zi};
-      const double r2 = dist2(d[0], d[1], d[2]);
-      if (!(r2 < R.rc2)) return;
-      const double inv2 = rcp_rn(r2);  // = 1.0 / r2, correctly rounded
-      const double s6 = inv2 * inv2 * inv2;
-      double rf = s6 * __builtin_fma(48.0, s6, -24.0);
-      const double t = 4.0 * s6;
-      double u = __builtin_fma(t, s6, -t) - R.shift;
-      if (SF) {
-        const double r = __builtin_sqrt(r2);
-        rf = __builtin_fma(-r, R.force_shift, rf);
-        u = __builtin_fma(r - R.rc, R.force_shift, u);
-      }
-      pe += 0.5 * u;
-      const double q = rf * inv2;
-      double w[3];
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        w[a] = (0.5 * d[a]) * d[a] * q;
-        total[a] += w[a];
-      }
-      const double lo = zw + (d[2] < 0.0 ? d[2] : 0.0);
-      const double hi = zw + (d[2] > 0.0 ? d[2] : 0.0);
-      const double length = hi - lo;
-      if (length < 1e-6 * width) {
-        win.add((int)home - hb, (int)home, ibins, w, 1.0, sink);
-        return;
-      }
-      int b = (int)floor(lo * iw);
-      double left = 1.0;
-      // A segment shorter than the box crosses at most bins + 1 slabs.
-      for (uint32_t walk = 0; walk < bins + 2u; walk++) {
-        const bool last = (double)(b + 1) * width >= hi;
-        const double start = lo > (double)b * width ? lo : (double)b * width;
-        const double end = hi < (double)(b + 1) * width ? hi : (double)(b + 1) * width;
-        double share = last ? left : (end - start) / length;
-        share = share > 0.0 ? share : 0.0;
-        left -= share;
-        win.add(b - hb, b, ibins, w, share, sink);
-        if (last) break;
-        b++;
-      }
-    });
-    // the window's sums, to the slabs below, at and above the atom's
-#pragma unroll
-    for (int kk = 0; kk < 3; kk++) {
-      const uint32_t slab = (uint32_t)((((hb - 1 + kk) % ibins) + ibins) % ibins);
-#pragma unroll
-      for (int a = 0; a < 3; a++) sink.add(slab * kProfileSums + 4u + (uint32_t)a, win.w[kk][a]);
-    }
-    sink.add(home * kProfileSums + 7u, pe);
-#pragma unroll
-    for (int a = 0; a < 3; a++) whole[a] += to_fixed(total[a], kProfileOne);
-  }
-}
 
 // A pair's potential u and q = rF / r^2 (R10, FP64 in both forms).
 template <bool SF>
@@ -2112,29 +2054,148 @@ __device__ __forceinline__ void profile_pair_terms(const Replica& R, double r2, 
 // in slab hb) to z + dz crosses, in proportion to the length inside each,
 // the last slab taking what is left (R10): into the atom's window sums, or
 // to the profile at once for a slab outside them.
-__device__ __forceinline__ void walk_shares(double zw, double dz, int hb, int home, double width, double iw,
-                                            uint32_t bins, const double w[3], SlabWindow& win,
-                                            const ProfileSink& sink) {
+// SMALL: every |w_a| of the wave is below kMagicMost. The loop's body is what the
+// profile costs (the lanes of a wave walk together, ~11 slabs where a pair crosses
+// 5 on average), so it holds only the share and the far slabs' adds, and the
+// window's three shares are picked out of it and added once.
+template <bool SMALL, class Sink>
+__device__ __forceinline__ void walk_slabs(double zw, double dz, int hb, int home, double width, double iw,
+                                           uint32_t bins, const double w[3], SlabWindow& win,
+                                           const Sink& sink) {
   const int ibins = (int)bins;
+  double dn = 0.0, own = 0.0, up = 0.0;
+  auto give = [&](int b, double share) {
+    const int k = b - hb;
+    dn = k == -1 ? share : dn;
+    own = k == 0 ? share : own;
+    up = k == 1 ? share : up;
+    if (k < -1 || k > 1) {
+      int slab = b < 0 ? b + ibins : (b >= ibins ? b - ibins : b);
+      if (__builtin_expect(slab < 0 || slab >= ibins, 0)) slab = ((b % ibins) + ibins) % ibins;
+      sink.template add_virial<SMALL>((uint32_t)slab, w, share);
+    }
+  };
   const double lo = zw + (dz < 0.0 ? dz : 0.0);
   const double hi = zw + (dz > 0.0 ? dz : 0.0);
   const double length = hi - lo;
   if (length < 1e-6 * width) {
-    win.add(home - hb, home, ibins, w, 1.0, sink);
-    return;
+    give(home, 1.0);
+  } else {
+    const double y = rcp_estimate(length);  // every share is a quotient by it
+    int b = (int)floor(lo * iw);
+    double left = 1.0, edge = (double)b * width;
+    // A segment shorter than the box crosses at most bins + 1 slabs.
+    for (uint32_t walk = 0; walk < bins + 2u; walk++) {
+      const double next = (double)(b + 1) * width;
+      const bool last = next >= hi;
+      const double start = lo > edge ? lo : edge;
+      const double end = hi < next ? hi : next;
+      double share = last ? left : div_rn(end - start, length, y);
+      share = share > 0.0 ? share : 0.0;
+      left -= share;
+      give(b, share);
+      if (last) break;
+      b++;
+      edge = next;
+    }
   }
-  int b = (int)floor(lo * iw);
-  double left = 1.0;
-  for (uint32_t walk = 0; walk < bins + 2u; walk++) {
-    const bool last = (double)(b + 1) * width >= hi;
-    const double start = lo > (double)b * width ? lo : (double)b * width;
-    const double end = hi < (double)(b + 1) * width ? hi : (double)(b + 1) * width;
-    double share = last ? left : (end - start) / length;
-    share = share > 0.0 ? share : 0.0;
-    left -= share;
-    win.add(b - hb, b, ibins, w, share, sink);
-    if (last) break;
-    b++;
+  win.add(w, dn, own, up);
+}
+
+template <class Sink>
+__device__ __forceinline__ void walk_shares(double zw, double dz, int hb, int home, double width, double iw,
+                                            uint32_t bins, const double w[3], SlabWindow& win,
+                                            const Sink& sink) {
+  const double most = __builtin_fmax(__builtin_fabs(w[0]), __builtin_fmax(__builtin_fabs(w[1]), __builtin_fabs(w[2])));
+  if (__builtin_amdgcn_ballot_w64(!(most < kMagicMost)) == 0ull)
+    walk_slabs<true>(zw, dz, hb, home, width, iw, bins, w, win, sink);
+  else
+    walk_slabs<false>(zw, dz, hb, home, width, iw, bins, w, win, sink);
+}
+
+// One brick's home atoms for slabs narrower than a cutoff: every pair's walk.
+// The list is read an octet at a time and the positions a pair ahead, so that a
+// walk runs while the next pair's LDS reads are in flight. us a sample, before and
+// now: eight slabs of 15,600 atoms, 240 slabs 720 / 450; 524,309 atoms, 200 slabs
+// 451 / 401; 3377 atoms, 80 slabs 184 / 127.
+template <bool SF, class L, bool LDS>
+__device__ __forceinline__ void profile_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
+                                             bool staged, const ProfileSink<L, LDS>& sink, long long whole[3]) {
+  const uint32_t bins = R.prof_bins;
+  const double width = R.bin_width;
+  const double iw = 1.0 / width;  // slab of z: floor(z iw)
+  const int ibins = (int)bins;
+  const uint32_t H = S.hoff[home_cells(g)];
+  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
+    const Home at = home_atom(g, S, h);
+    const uint32_t i = at.slot;
+    double xi, yi, zi;
+    staged_pos(R, S, staged, at.e, B.x, B.y, B.z, xi, yi, zi);
+    const double zw = wrap_one(zi, R.box[2]);
+    const int hb = (int)floor(zw * iw);  // the slab the shares are counted from
+    const uint32_t home = (uint32_t)(hb < 0 ? 0 : (hb > ibins - 1 ? ibins - 1 : hb));
+    sink.atom(home, 0u, to_fixed(1.0, kProfileOne));
+    const double v[3] = {B.vx[i], B.vy[i], B.vz[i]};
+#pragma unroll
+    for (uint32_t a = 0; a < 3u; a++) sink.atom(home, 1u + a, to_fixed(v[a] * v[a], kProfileOne));
+    double pe = 0.0, total[3] = {0.0, 0.0, 0.0};
+    SlabWindow win;
+    win.clear();
+    const uint32_t cnt = B.nbr_count[i];
+    const uint16_t* lst = B.nbr + list_base(R, i - R.atom_off);
+    auto pair = [&](double dx, double dy, double dz) {
+      const double r2 = dist2(dx, dy, dz);
+      if (!(r2 < R.rc2)) return;
+      double u, q;
+      profile_pair_terms<SF>(R, r2, u, q);
+      pe += 0.5 * u;
+      const double w[3] = {(0.5 * dx) * dx * q, (0.5 * dy) * dy * q, (0.5 * dz) * dz * q};
+#pragma unroll
+      for (int a = 0; a < 3; a++) total[a] += w[a];
+      walk_shares(zw, dz, hb, (int)home, width, iw, bins, w, win, sink);
+    };
+    if (staged) {
+      const uint32_t no = (cnt + 7u) / 8u;
+      const uint32_t last_octet = no > 0u ? no - 1u : 0u;
+      u32x4 cur = load_octet(lst, 0u, last_octet), nxt = load_octet(lst, 1u, last_octet);
+      auto take = [&](double p[3]) {  // the position of the octet's next entry
+        const uint32_t off = cur.x & 0xffffu;  // 8 e
+        p[0] = *(const double*)((const char*)S.x + off);
+        p[1] = *(const double*)((const char*)S.y + off);
+        p[2] = *(const double*)((const char*)S.z + off);
+        cur.x = (cur.x >> 16) | (cur.y << 16);
+        cur.y = (cur.y >> 16) | (cur.z << 16);
+        cur.z = (cur.z >> 16) | (cur.w << 16);
+        cur.w >>= 16;
+      };
+      double p[3] = {kFar, kFar, kFar};
+      if (no) take(p);
+      for (uint32_t k = 0; k < 8u * no; k++) {
+        const double x = p[0], y = p[1], z = p[2];
+        if ((k & 7u) == 7u) {
+          cur = nxt;
+          nxt = load_octet(lst, (k + 1u) / 8u + 1u, last_octet);
+        }
+        take(p);  // past the last octet: its entries again, never summed
+        pair(x - xi, y - yi, z - zi);
+      }
+    } else {
+      each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
+        double xj, yj, zj;
+        staged_pos(R, S, false, list_index(entry, false), B.x, B.y, B.z, xj, yj, zj);
+        pair(xj - xi, yj - yi, zj - zi);
+      });
+    }
+    // the window's sums, to the slabs below, at and above the atom's
+#pragma unroll
+    for (int kk = 0; kk < 3; kk++) {
+      const uint32_t slab = (uint32_t)((((hb - 1 + kk) % ibins) + ibins) % ibins);
+#pragma unroll
+      for (uint32_t a = 0; a < 3u; a++) sink.virial(slab, a, to_fixed(win.w[kk][a], kProfileOne));
+    }
+    sink.atom(home, 7u, to_fixed(pe, kProfileOne));
+#pragma unroll
+    for (int a = 0; a < 3; a++) whole[a] += to_fixed(total[a], kProfileOne);
   }
 }
 
@@ -2154,7 +2215,7 @@ template <bool SF, class L>
 __device__ __forceinline__ void wide_pairs_staged(const Replica& R, const Stage<L>& S, const uint16_t* lst,
                                                   uint32_t cnt, double xi, double yi, double zi, double zw, int hb,
                                                   int home, double width, double iw, uint32_t bins,
-                                                  const ProfileSink& sink, double& pe, double total[3],
+                                                  const ProfileSink<L, false>& sink, double& pe, double total[3],
                                                   SlabWindow& win) {
   const double tiny_length = 1e-6 * width;
   const uint32_t no = (cnt + 7u) / 8u;
@@ -2197,7 +2258,7 @@ __device__ __forceinline__ void wide_pairs_staged(const Replica& R, const Stage<
       const bool last2 = (double)(b + 2) * width >= hi;
       const double start = lo > bw ? lo : bw;
       const double end = hi < e1 ? hi : e1;
-      double s1 = last1 ? 1.0 : (end - start) / length;
+      double s1 = last1 ? 1.0 : div_rn(end - start, length, rcp_estimate(length));
       s1 = s1 > 0.0 ? s1 : 0.0;
       double s2 = 1.0 - s1;
       s2 = s2 > 0.0 ? s2 : 0.0;
@@ -2245,7 +2306,7 @@ __device__ __forceinline__ void profile_part_wide(const Buffers& B, const Replic
   const double width = R.bin_width;
   const double iw = 1.0 / width;  // slab of z: floor(z iw)
   const int ibins = (int)bins;
-  const ProfileSink direct{nullptr, prof, false};
+  const ProfileSink<L, false> direct{nullptr, prof};
   const uint32_t H = S.hoff[home_cells(g)];
   const uint32_t lane = threadIdx.x & 63u;
   // one wave-wide sum per slot of sum q, the lanes' values from `value`
@@ -2293,7 +2354,7 @@ __device__ __forceinline__ void profile_part_wide(const Buffers& B, const Replic
       for (int q = 0; q < 4; q++) send(hmin, q, [&](int rs) { return active && hslot == rs ? item[q] : 0ll; });
     } else if (active) {
 #pragma unroll
-      for (int q = 0; q < 4; q++) direct.add(home * kProfileSums + (uint32_t)q, item[q]);
+      for (int q = 0; q < 4; q++) direct.atom(home, (uint32_t)q, item[q]);
     }
     SlabWindow win;
     win.clear();
@@ -2345,27 +2406,43 @@ __device__ __forceinline__ void profile_part_wide(const Buffers& B, const Replic
           return x;
         });
     } else if (active) {
-      direct.add(home * kProfileSums + 7u, pe_fixed);
+      direct.atom(home, 7u, pe_fixed);
 #pragma unroll
       for (int kk = 0; kk < 3; kk++) {
         const uint32_t slab = (uint32_t)((((hb - 1 + kk) % ibins) + ibins) % ibins);
 #pragma unroll
-        for (int a = 0; a < 3; a++) direct.add(slab * kProfileSums + 4u + (uint32_t)a, wf[kk][a]);
+        for (int a = 0; a < 3; a++) direct.virial(slab, (uint32_t)a, wf[kk][a]);
       }
     }
   }
 }
 
 // Adds the workgroup's sums of one brick to the replica's profile.
-template <class L>
-__device__ __forceinline__ void profile_flush(const ProfileSink& sink, uint32_t bins, const long long whole[3]) {
-  const uint32_t nsums = bins * kProfileSums + 3u;
+template <class L, bool LDS>
+__device__ __forceinline__ void profile_flush(const ProfileSink<L, LDS>& sink, uint32_t bins, const long long whole[3]) {
 #pragma unroll
-  for (int a = 0; a < 3; a++) sink.add(bins * kProfileSums + (uint32_t)a, whole[a]);
-  if (sink.use_lds) {
-    __syncthreads();
-    for (uint32_t k = threadIdx.x; k < nsums; k += L::kThreads)
-      if (sink.lds[k] != 0) atomicAdd((unsigned long long*)(sink.global + k), (unsigned long long)sink.lds[k]);
+  for (uint32_t a = 0; a < 3u; a++) {
+    const long long x = wave_sum_i64(whole[a]);
+    if ((threadIdx.x & 63u) != 0 || x == 0) continue;
+    if constexpr (LDS)
+      atomicAdd((unsigned long long*)&sink.lds->total[a], (unsigned long long)x);
+    else
+      atomicAdd((unsigned long long*)(sink.global + bins * kProfileSums + a), (unsigned long long)x);
+  }
+  if constexpr (!LDS) return;
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < bins * kProfileSums + 3u; k += L::kThreads) {
+    const uint32_t b = k / kProfileSums, q = k % kProfileSums;
+    long long x = 0;
+    if (b == bins) {
+      x = sink.lds->total[q];
+    } else if (q >= 4u && q < 7u) {
+#pragma unroll
+      for (uint32_t c = 0; c < ProfileBins<L>::kCopies; c++) x += sink.lds->w[q - 4u][b * ProfileBins<L>::kCopies + c];
+    } else {
+      x = sink.lds->atom[q == 7u ? 4u : q][b];
+    }
+    if (x != 0) atomicAdd((unsigned long long*)(sink.global + k), (unsigned long long)x);
   }
 }
 
@@ -2403,25 +2480,36 @@ __global__ void __launch_bounds__(L::kThreads, WIDE && !PARTS && !L::kSparse ? 4
     }
     return;
   }
-  __shared__ long long acc[WIDE ? 1 : kProfileLdsBins * kProfileSums + 3];
-  auto profile = [&](uint32_t gb, uint32_t code) {
-    const Brick brick = B.bricks[gb];
-    const Replica R = B.rep[brick.rep];
-    const uint32_t bins = R.prof_bins;
-    if (bins == 0) return;  // the whole workgroup together
-    const uint32_t nsums = bins * kProfileSums + 3u;
-    const ProfileSink sink{acc, B.profile + R.prof_off, bins <= kProfileLdsBins};
-    const Brick g = PARTS ? part_brick(brick, code, R) : brick;
-    if (PARTS) __syncthreads();  // the previous part is done with S and acc
-    if (sink.use_lds)
-      for (uint32_t k = threadIdx.x; k < nsums; k += L::kThreads) acc[k] = 0;
-    const bool staged = stage_brick(B, R, g, B.x, B.y, B.z, S);  // ends with a barrier
-    if (!PARTS && !staged && home_cells(g) > 1u && B.parts_on) return;  // cut into parts
-    long long whole[3] = {0, 0, 0};
-    profile_part<SF>(B, R, S, g, staged, sink, whole);
-    profile_flush<L>(sink, bins, whole);
-  };
   if constexpr (!WIDE) {
+    __shared__ ProfileBins<L> acc;
+    auto profile = [&](uint32_t gb, uint32_t code) {
+      const Brick brick = B.bricks[gb];
+      const Replica R = B.rep[brick.rep];
+      const uint32_t bins = R.prof_bins;
+      if (bins == 0) return;  // the whole workgroup together
+      const bool use_lds = bins <= kProfileLdsBins;
+      const Brick g = PARTS ? part_brick(brick, code, R) : brick;
+      if (PARTS) __syncthreads();  // the previous part is done with S and acc
+      if (use_lds) {
+        for (uint32_t k = threadIdx.x; k < bins * ProfileBins<L>::kCopies; k += L::kThreads)
+          acc.w[0][k] = acc.w[1][k] = acc.w[2][k] = 0;
+        for (uint32_t b = threadIdx.x; b < bins; b += L::kThreads)
+          acc.atom[0][b] = acc.atom[1][b] = acc.atom[2][b] = acc.atom[3][b] = acc.atom[4][b] = 0;
+        if (threadIdx.x < 3u) acc.total[threadIdx.x] = 0;
+      }
+      const bool staged = stage_brick(B, R, g, B.x, B.y, B.z, S);  // ends with a barrier
+      if (!PARTS && !staged && home_cells(g) > 1u && B.parts_on) return;  // cut into parts
+      long long whole[3] = {0, 0, 0};
+      if (use_lds) {
+        const ProfileSink<L, true> sink{&acc, B.profile + R.prof_off};
+        profile_part<SF>(B, R, S, g, staged, sink, whole);
+        profile_flush(sink, bins, whole);
+      } else {
+        const ProfileSink<L, false> sink{nullptr, B.profile + R.prof_off};
+        profile_part<SF>(B, R, S, g, staged, sink, whole);
+        profile_flush(sink, bins, whole);
+      }
+    };
     if constexpr (!PARTS) {
       const uint32_t gb = layout_first<L>(B) + dealt_index(blockIdx.x);
       if (gb < layout_end<L>(B)) profile(gb, 0u);
