@@ -23,27 +23,50 @@ namespace vlj {
 // Wave64 / workgroup helpers
 // ---------------------------------------------------------------------------
 
+// A value from the lane that one step of a scan over a wave reads, 0 where there
+// is none: DPP moves inside the vector unit, a few cycles each against the >100
+// of a shuffle through LDS. The steps: 1, 2, 4, 8 lanes back in a row of 16,
+// then a row's last lane to the next row, then lane 31 to the upper half. Every
+// lane of the wave is active.
+template <int STEP>
+__device__ __forceinline__ uint32_t lane_back(uint32_t v) {
+  constexpr int ctrl = STEP < 4 ? 0x110 + (1 << STEP) : STEP == 4 ? 0x142 : 0x143;  // row_shr:n, row_bcast:15, :31
+  constexpr int rows = STEP < 4 ? 0xf : STEP == 4 ? 0xa : 0xc;
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false);
+}
+template <int STEP>
+__device__ __forceinline__ unsigned long long lane_back(unsigned long long v) {
+  return (unsigned long long)lane_back<STEP>((uint32_t)(v >> 32)) << 32 | lane_back<STEP>((uint32_t)v);
+}
+
+// f over the wave, in every lane; f(0, v) = v.
+template <class F>
+__device__ __forceinline__ unsigned long long wave_all(unsigned long long v, F&& f) {
+  v = f(lane_back<0>(v), v);
+  v = f(lane_back<1>(v), v);
+  v = f(lane_back<2>(v), v);
+  v = f(lane_back<3>(v), v);
+  v = f(lane_back<4>(v), v);
+  v = f(lane_back<5>(v), v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+  return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63) << 32 | lo;
+}
+
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    unsigned long long o = __shfl_xor(v, off, 64);
-    v = o > v ? o : v;
-  }
-  return v;
+  return wave_all(v, [](unsigned long long o, unsigned long long x) { return o > x ? o : x; });
 }
 
 __device__ __forceinline__ long long wave_sum_i64(long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  return (long long)wave_all((unsigned long long)v, [](unsigned long long o, unsigned long long x) { return o + x; });
 }
 
-__device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v, int lane) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    uint32_t o = __shfl_up(v, off, 64);
-    if (lane >= off) v += o;
-  }
+__device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
+  v += lane_back<0>(v);
+  v += lane_back<1>(v);
+  v += lane_back<2>(v);
+  v += lane_back<3>(v);
+  v += lane_back<4>(v);
+  v += lane_back<5>(v);
   return v;
 }
 
@@ -507,7 +530,7 @@ __global__ void __launch_bounds__(kChainThreads) k_chain(Buffers B) {
     n[k] = k < per && c < R.total_cells ? first[c] : 0u;
     sum += n[k];
   }
-  const uint32_t incl = wave_incl_scan_u32(sum, (int)(t & 63u));
+  const uint32_t incl = wave_incl_scan_u32(sum);
   if ((t & 63u) == 63u) wsum[t >> 6] = incl;
   __syncthreads();
   uint32_t run = incl - sum;
@@ -570,7 +593,7 @@ __global__ void __launch_bounds__(kBlock) k_scan(Buffers B) {
       local += v[k];
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t incl = wave_incl_scan_u32(local, lane);
+    uint32_t incl = wave_incl_scan_u32(local);
     if (lane == 63) wsum[wave] = incl;
     __syncthreads();
     uint32_t before = 0, total = 0;
@@ -774,6 +797,12 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 // workgroup calls it. Returns whether the positions were staged (the
 // neighbourhood holds at most L::kStageMax atoms). `via`, in a rebuild: the
 // positions are still in the old order and not wrapped yet, slot j's at via[j].
+// A chain of dependent loads (brick, replica, cells, positions), ~0.7 us each,
+// that a small brick cannot hide; what lies between them is kept short: scans
+// by DPP moves, home atoms numbered in the same pass as the staged ones, no
+// integer division a cell. us/step before (shuffles, a third scan by one wave,
+// 8 divisions a cell) / with: 1000 atoms 20.1 / 19.2, 50,653 36.9 / 36.0, FCC-1M
+// 196 / 191 (FP32 190 / 184), the 16-replica batch 314 / 306.
 template <class L>
 __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, const double* X, const double* Y,
                             const double* Z, Stage<L>& S, const uint32_t* via = nullptr) {
@@ -781,54 +810,74 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
   __builtin_amdgcn_s_setprio(VLJ_STAGE_PRIO);
 #endif
   const int nx = (int)R.cells[0], ny = (int)R.cells[1], nz = (int)R.cells[2];
-  const int c0 = (int)g.cell0;
-  const int cx0 = c0 % nx, cy0 = (c0 / nx) % ny, cz = c0 / (nx * ny);
+  const uint32_t row0 = g.cell0 / R.cells[0];
+  const int cx0 = (int)(g.cell0 - row0 * R.cells[0]), cz = (int)(row0 / R.cells[1]), cy0 = (int)row0 - cz * ny;
   const uint32_t sx = g.gx + 2u, sy = g.gy + 2u;
   const uint32_t ns = (g.gz + 2u) * sy * sx;  // at most kStageCells
   const uint32_t t = threadIdx.x;
+  // (c + 0.5) / n is at least 0.5 / n from a whole number: the estimates below
+  // round down to c / n for every staged cell
+  static_assert(kStageCells <= 4096, "exact in FP32");
+  const float isx = __builtin_amdgcn_rcpf((float)sx), isy = __builtin_amdgcn_rcpf((float)sy);
   // thread t stages the kCellsPerThread consecutive cells from t * kCellsPerThread
   constexpr uint32_t kCPT = (uint32_t)L::kCellsPerThread;
   uint32_t n_c[kCPT], st_c[kCPT];
+  bool home_c[kCPT];
   bool shifted_cell = false;  // a cell of this thread is a periodic image
 #pragma unroll
   for (uint32_t h = 0; h < kCPT; h++) {
     const uint32_t c = kCPT * t + h;
     n_c[h] = 0u;
     st_c[h] = 0u;
+    home_c[h] = false;
     if (c < ns) {
-      const int xx = (int)(c % sx), yy = (int)((c / sx) % sy), dz = (int)(c / (sx * sy));
-      const int ux = cx0 - 1 + xx, uy = cy0 - 1 + yy, uz = cz - 1 + dz;  // unwrapped
-      const int cx = (ux + nx) % nx, cy = (uy + ny) % ny, ccz = (uz + nz) % nz;
-      const uint32_t cell = R.cell_off + (uint32_t)((ccz * ny + cy) * nx + cx);
-      st_c[h] = B.cell_start[cell];
-      n_c[h] = B.cell_n[cell];
+      const uint32_t row = (uint32_t)(((float)c + 0.5f) * isx), xx = c - row * sx;
+      const uint32_t dz = (uint32_t)(((float)row + 0.5f) * isy), yy = row - dz * sy;
+      const int ux = cx0 - 1 + (int)xx, uy = cy0 - 1 + (int)yy, uz = cz - 1 + (int)dz;  // unwrapped, from -1 to the count
       // image of the cell seen from the brick (R4)
       const int ix = ux < 0 ? -1 : (ux >= nx ? 1 : 0);
       const int iy = uy < 0 ? -1 : (uy >= ny ? 1 : 0);
       const int iz = uz < 0 ? -1 : (uz >= nz ? 1 : 0);
+      const int cx = ux - ix * nx, cy = uy - iy * ny, ccz = uz - iz * nz;
+      const uint32_t cell = R.cell_off + (uint32_t)((ccz * ny + cy) * nx + cx);
+      st_c[h] = B.cell_start[cell];
+      n_c[h] = B.cell_n[cell];
+      home_c[h] = xx - 1u < g.gx && yy - 1u < g.gy && dz - 1u < g.gz;
       S.image[c] = (uint8_t)((ix + 1) | (iy + 1) << 2 | (iz + 1) << 4);
       shifted_cell = shifted_cell || ix != 0 || iy != 0 || iz != 0;
     }
   }
-  // exclusive scan of the staged counts over the workgroup; each wave's
-  // total carries in its top bit whether the wave staged an image cell
-  __shared__ uint32_t wtot[L::kThreads / 64];
-  uint32_t n_t = 0;
+  // exclusive scans over the workgroup of the staged counts and of the home
+  // cells' and their counts (home cells come in home order, hz, hy outer, hx
+  // inner); each wave's staged total carries in its top bit whether the wave
+  // staged an image cell
+  __shared__ uint32_t wtot[L::kThreads / 64], whome[L::kThreads / 64], wcells[L::kThreads / 64];
+  uint32_t n_t = 0, h_t = 0, k_t = 0;
 #pragma unroll
-  for (uint32_t h = 0; h < kCPT; h++) n_t += n_c[h];
+  for (uint32_t h = 0; h < kCPT; h++) {
+    n_t += n_c[h];
+    h_t += home_c[h] ? n_c[h] : 0u;
+    k_t += home_c[h] ? 1u : 0u;
+  }
   const int lane = t & 63, wave = t >> 6;
-  const uint32_t incl = wave_incl_scan_u32(n_t, lane);
+  const uint32_t incl = wave_incl_scan_u32(n_t), hincl = wave_incl_scan_u32(h_t), kincl = wave_incl_scan_u32(k_t);
   const bool wave_shifted = __builtin_amdgcn_ballot_w64(shifted_cell) != 0ull;
-  if (lane == 63) wtot[wave] = incl | (wave_shifted ? 0x80000000u : 0u);
+  if (lane == 63) {
+    wtot[wave] = incl | (wave_shifted ? 0x80000000u : 0u);
+    whome[wave] = hincl;
+    wcells[wave] = kincl;
+  }
   __syncthreads();
-  uint32_t before = 0, shifted_any = 0;
+  uint32_t before = 0, hbefore = 0, kbefore = 0, shifted_any = 0;
 #pragma unroll
   for (int w = 0; w < L::kThreads / 64; w++) {
     const uint32_t x = wtot[w];
     before += w < wave ? x & 0x7fffffffu : 0u;
+    hbefore += w < wave ? whome[w] : 0u;
+    kbefore += w < wave ? wcells[w] : 0u;
     shifted_any |= x >> 31;
   }
-  uint32_t run = before + incl - n_t;
+  uint32_t run = before + incl - n_t, hrun = hbefore + hincl - h_t, krun = kbefore + kincl - k_t;
 #pragma unroll
   for (uint32_t h = 0; h < kCPT; h++) {
     const uint32_t c = kCPT * t + h;
@@ -839,6 +888,10 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
       // below kStageMax are indexed), known here without reading S.off back
       const uint32_t end = run + n_c[h] < (uint32_t)L::kStageMax ? run + n_c[h] : (uint32_t)L::kStageMax;
       for (uint32_t m = (run + kCoarse - 1u) / kCoarse; m * kCoarse < end; m++) S.coarse[m] = (uint16_t)c;
+      if (home_c[h]) {
+        S.hoff[krun++] = hrun;
+        hrun += n_c[h];
+      }
     }
     run += n_c[h];
   }
@@ -846,19 +899,9 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
     S.off[ns] = before + incl;
     S.total = before + incl;
     S.ns = ns;
+    S.hoff[kbefore + kincl] = hbefore + hincl;
   }
   __syncthreads();
-  if (t < 64u) {  // home atoms, home cell by home cell (hz, hy outer, hx inner): a scan over wave 0
-    const uint32_t nh = home_cells(g);  // at most kHomeCells = 64
-    uint32_t n = 0;
-    if (t < nh) {
-      const uint32_t hs = staged_cell(g, t / (g.gx * g.gy) + 1u, (t / g.gx) % g.gy + 1u, t % g.gx + 1u);
-      n = S.off[hs + 1u] - S.off[hs];
-    }
-    const uint32_t incl = wave_incl_scan_u32(n, lane);
-    if (t < nh) S.hoff[t] = incl - n;
-    if (t + 1u == nh) S.hoff[nh] = incl;
-  }
   const uint32_t total = S.total;
   const bool staged = total <= (uint32_t)L::kStageMax;
   if (staged) {
@@ -1042,7 +1085,7 @@ template <int THREADS>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* total) {
   __shared__ uint32_t wsum[THREADS / 64];
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t incl = wave_incl_scan_u32(v, (int)lane);
+  const uint32_t incl = wave_incl_scan_u32(v);
   __syncthreads();  // earlier readers of wsum are done
   if (lane == 63u) wsum[wave] = incl;
   __syncthreads();
@@ -1267,7 +1310,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
   const uint32_t each = (H + (uint32_t)(L::kThreads / 64) - 1u) / (uint32_t)(L::kThreads / 64);
   const uint32_t piece = each < 4u ? 4u : (each < kPiece ? each : kPiece);
   const uint32_t pieces = (hn + piece - 1u) / piece;
-  const uint32_t pincl = wave_incl_scan_u32(pieces, (int)lane);
+  const uint32_t pincl = wave_incl_scan_u32(pieces);
   const uint32_t pv = pincl - pieces;  // lanes past the home cells: the item count
   const uint32_t n_items = readlane_u32(pincl, 63);
   for (;;) {
@@ -1293,7 +1336,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
       rs = S.off[sc];
       rl = S.off[sc + 3u] - rs;
     }
-    const uint32_t rincl = wave_incl_scan_u32(rl, (int)lane);
+    const uint32_t rincl = wave_incl_scan_u32(rl);
     const uint32_t rdv = rs + rl - rincl;
     uint32_t rend[9], rdelta[9];
 #pragma unroll
