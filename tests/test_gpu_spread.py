@@ -91,3 +91,21 @@ def test_forms_change_around_the_decision(oracle, lj):
             ref.run(steps)
             assert list(sim.measure_now().raw) == list(ref.measure().raw)
             np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
+
+
+@pytest.mark.parametrize("thermostat", [0, 1])  # drift-ahead steps, which swap the position sets, and plain ones
+def test_calls_of_any_length_are_the_same_run(lj, thermostat):
+    def simulation():
+        parts, side = lj.fcc_count_array(1100, 0.8442, 1.0, 7)
+        th = lj.Langevin(1.0, 1.0, 5) if thermostat else None
+        return lj.LennardJones(parts, lj.Settings([side] * 3, 2.5, 0.004, skin=0.3, thermostat=th))
+    one, many = simulation(), simulation()
+    lengths = (1, 2, 3, 1, 4, 7, 8, 5, 15, 16, 17, 31, 6, 12, 1)
+    for steps in lengths:
+        many.run(steps)
+    for _ in range(sum(lengths)):
+        one.run(1)
+    assert list(one.measure_now().raw) == list(many.measure_now().raw)
+    assert one.measure_now().step == many.measure_now().step == sum(lengths)
+    np.testing.assert_array_equal(one.debug_state()[0], many.debug_state()[0])
+    np.testing.assert_array_equal(one.debug_state()[1], many.debug_state()[1])

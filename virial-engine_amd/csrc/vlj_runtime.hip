@@ -2,7 +2,7 @@
 //
 // The handle owns one HIP stream, every device buffer, a 3-slot pinned
 // read-back ring for measurements and the step sequence captured as
-// hipGraphs (one step and kGraphSteps steps). It replaces the wgpu-side host
+// hipGraphs (of 1, 2, 4, 8 and 16 steps). It replaces the wgpu-side host
 // of crates/virial-particles/src/lennard_jones.rs:443-1375.
 #include <hip/hip_runtime.h>
 
@@ -22,7 +22,13 @@ using namespace vlj;
 namespace {
 
 constexpr int kRing = 3;         // read-back slots (lennard_jones.rs:320)
-constexpr uint32_t kGraphSteps = 16;
+// Steps are captured in graphs of 2^k of them, k below kGraphs, each on its
+// first use: a call for few steps between two samples is one or two launches
+// (a graph launch takes ~10 us on the host and leaves a gap of several us).
+// 16,384 atoms, a heat-current sample every second step, us per sample with
+// graphs of 1 and 16 only / these: 75.6 / 65.8; a profile sample every 20 steps,
+// 4096 atoms: 437 / 428.
+constexpr uint32_t kGraphs = 5;
 // Brick planner. Bricks are planned to stage at most kDefaultFill of the
 // LDS staging limit until the tuner has measured the candidates kTuneFills
 // (kTuneSteps steps each) on the handle's own state; a handle of at least
@@ -116,7 +122,7 @@ struct vlj_sim {
   std::vector<void*> allocations;
   Ring ring[kRing];
   // captured steps, for each orientation of the position sets
-  hipGraphExec_t graph1[2] = {nullptr, nullptr}, graphN[2] = {nullptr, nullptr};
+  hipGraphExec_t graphs[2][kGraphs] = {};
   // The drift-ahead form (every replica NVE): a step's force launch also
   // drifts the positions of the next step into the second position set
   // (B.x2); `ahead` says it holds them. Each step that uses them swaps the
@@ -357,8 +363,8 @@ void free_device(vlj_sim* s, void* p) {
 void free_all(vlj_sim* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   for (int k = 0; k < 2; k++) {
-    if (s->graph1[k]) (void)hipGraphExecDestroy(s->graph1[k]);
-    if (s->graphN[k]) (void)hipGraphExecDestroy(s->graphN[k]);
+    for (hipGraphExec_t g : s->graphs[k])
+      if (g) (void)hipGraphExecDestroy(g);
   }
   for (auto& r : s->ring) {
     if (r.slots) (void)hipHostFree(r.slots);
@@ -449,9 +455,10 @@ int enqueue_step(vlj_sim* s, hipEvent_t* around_force = nullptr) {
 void drop_graphs(vlj_sim* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   for (int k = 0; k < 2; k++) {
-    if (s->graph1[k]) (void)hipGraphExecDestroy(s->graph1[k]);
-    if (s->graphN[k]) (void)hipGraphExecDestroy(s->graphN[k]);
-    s->graph1[k] = s->graphN[k] = nullptr;
+    for (hipGraphExec_t& g : s->graphs[k]) {
+      if (g) (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
   }
 }
 
@@ -1167,14 +1174,17 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   return VLJ_OK;
 }
 
-// The captured steps for the present orientation of the position sets (the
-// drift-ahead form swaps them every step: one pair of graphs each way).
-int ensure_graphs(vlj_sim* s) {
-  const int o = s->orient;
-  int rc = VLJ_OK;
-  if (!s->graph1[o]) rc = capture(s, 1, &s->graph1[o]);
-  if (rc == VLJ_OK && !s->graphN[o]) rc = capture(s, kGraphSteps, &s->graphN[o]);
-  return rc;
+// 2^k captured steps for the present orientation of the position sets (the
+// drift-ahead form swaps them every step: one set of graphs each way).
+int replay(vlj_sim* s, uint32_t k) {
+  hipGraphExec_t& g = s->graphs[s->orient][k];
+  if (!g) {
+    const int rc = capture(s, 1u << k, &g);
+    if (rc != VLJ_OK) return rc;
+  }
+  HIP_TRY(s, hipGraphLaunch(g, s->stream));
+  if (k == 0 && drift_ahead(s)) flip_positions(s);  // an even count: the sets end as they began
+  return VLJ_OK;
 }
 
 int enqueue_steps(vlj_sim* s, uint64_t steps) {
@@ -1199,19 +1209,11 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
     if (rc != VLJ_OK) return rc;
     left--;
   }
-  while (left >= kGraphSteps) {
-    rc = ensure_graphs(s);
-    if (rc != VLJ_OK) return rc;
-    HIP_TRY(s, hipGraphLaunch(s->graphN[s->orient], s->stream));  // an even count: the sets end as they began
-    left -= kGraphSteps;
-  }
-  while (left > 0) {
-    rc = ensure_graphs(s);
-    if (rc != VLJ_OK) return rc;
-    HIP_TRY(s, hipGraphLaunch(s->graph1[s->orient], s->stream));
-    if (drift_ahead(s)) flip_positions(s);
-    left--;
-  }
+  for (uint32_t k = kGraphs; k-- > 0;)
+    for (; left >= 1ull << k; left -= 1ull << k) {
+      rc = replay(s, k);
+      if (rc != VLJ_OK) return rc;
+    }
   // what the replayed steps leave: drifted positions in B.x2 after
   // drift-ahead steps, none after the others (which use B.x2 as scratch)
   if (steps > 0) {
