@@ -109,3 +109,33 @@ def test_calls_of_any_length_are_the_same_run(lj, thermostat):
     assert one.measure_now().step == many.measure_now().step == sum(lengths)
     np.testing.assert_array_equal(one.debug_state()[0], many.debug_state()[0])
     np.testing.assert_array_equal(one.debug_state()[1], many.debug_state()[1])
+
+
+@pytest.mark.parametrize("n,box,cutoff,shifted,precision", [
+    (343, 8.6, 2.5, True, 0),     # one block a brick: its crew is the workgroup
+    (343, 8.6, 2.5, False, 1),
+    (344, 11.0, 2.5, False, 0),   # ... and an atom with no neighbour at all
+    (729, 15.0, 4.5, False, 0),   # a droplet: bricks of one to three blocks, lists of up to ~40 octets
+    (729, 15.0, 4.5, True, 1),
+    (1728, 15.0, 4.5, True, 0),    # 1728 staged atoms leave no room for crews
+    (1728, 15.0, 4.5, False, 1),
+])
+def test_crews_against_the_oracle(oracle, lj, n, box, cutoff, shifted, precision):
+    edge = round(n ** (1.0 / 3.0))
+    grid = np.resize(np.stack(np.meshgrid(*[np.arange(edge)] * 3, indexing="ij"), -1).reshape(-1, 3), (n, 3))
+    rng = np.random.default_rng(17)
+    pos = np.ascontiguousarray((grid - 0.5 * (edge - 1)) * 1.12 + 0.5 * box + rng.uniform(-0.03, 0.03, (n, 3)))
+    if n == 344:
+        pos[-1] = 0.1
+    vel = np.ascontiguousarray(rng.normal(0.0, 0.7, (n, 3)))
+    vel -= vel.mean(axis=0)
+    sim = lj.LennardJones((pos, vel), lj.Settings([box] * 3, cutoff, 0.003, skin=0.3, shifted_force=shifted,
+                                                  precision=precision))
+    ref = oracle.Sim(pos, vel, [box] * 3, cutoff=cutoff, skin=0.3, dt=0.003, shifted_force=shifted,
+                     precision=precision)
+    for steps in (1, 40):
+        sim.run(steps)
+        ref.run(steps)
+        assert list(sim.measure_now().raw) == list(ref.measure().raw)
+        np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
+        np.testing.assert_array_equal(sim.debug_state()[1], ref.state()[1])

@@ -155,6 +155,7 @@ struct Buffers {
   uint16_t* parts;            // per brick: kHomeCells packed parts
   uint32_t* cut_groups;       // per group of kCutGroup bricks: bricks cut
   uint32_t n_atom_blocks, n_scan_blocks, n_sort_blocks, n_bricks, n_replicas, n_dense;
+  uint32_t crews;  // the dense bricks are small: crews of waves share their atoms' pairs
   // 1: a brick whose neighbourhood outgrows LDS is cut into parts, which the
   // PARTS launches after each brick launch take; 0: no PARTS launches, and
   // such a brick runs whole, its positions read through the cell tables

@@ -803,9 +803,14 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 // integer division a cell. us/step before (shuffles, a third scan by one wave,
 // 8 divisions a cell) / with: 1000 atoms 20.1 / 19.2, 50,653 36.9 / 36.0, FCC-1M
 // 196 / 191 (FP32 190 / 184), the 16-replica batch 314 / 306.
-template <class L>
+struct NoCrew {
+  __device__ __forceinline__ void cells_known() {}
+  __device__ __forceinline__ void loads_done() {}
+};
+
+template <class L, class Crew = NoCrew>
 __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, const double* X, const double* Y,
-                            const double* Z, Stage<L>& S, const uint32_t* via = nullptr) {
+                            const double* Z, Stage<L>& S, const uint32_t* via = nullptr, Crew&& crew = Crew()) {
 #if VLJ_STAGE_PRIO
   __builtin_amdgcn_s_setprio(VLJ_STAGE_PRIO);
 #endif
@@ -902,6 +907,7 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
     S.hoff[kbefore + kincl] = hbefore + hincl;
   }
   __syncthreads();
+  crew.cells_known();
   const uint32_t total = S.total;
   const bool staged = total <= (uint32_t)L::kStageMax;
   if (staged) {
@@ -955,6 +961,7 @@ __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, 
     }
     if (t == 0) S.x[L::kListPad] = S.y[L::kListPad] = S.z[L::kListPad] = kFar;
   }
+  crew.loads_done();
   __syncthreads();
 #if VLJ_STAGE_PRIO
   __builtin_amdgcn_s_setprio(0);
@@ -1622,9 +1629,9 @@ static_assert(8 % kPairs == 0, "an octet is whole groups");
 __device__ __forceinline__ void side_by_side() { __builtin_amdgcn_sched_barrier(0); }
 
 template <bool SF>
-__device__ __forceinline__ void pairs_force(const Replica& R, const double* dx, const double* dy, const double* dz,
-                                            PairAcc& a) {
-  double r2[kPairs], q[kPairs], y[kPairs], e[kPairs], g[kPairs];
+__device__ __forceinline__ void pairs_factor(const Replica& R, const double* dx, const double* dy, const double* dz,
+                                             double* g) {
+  double r2[kPairs], q[kPairs], y[kPairs], e[kPairs];
   bool hit[kPairs];
 #pragma unroll
   for (int p = 0; p < kPairs; p++) {
@@ -1671,6 +1678,13 @@ __device__ __forceinline__ void pairs_force(const Replica& R, const double* dx, 
 #pragma unroll
   for (int p = 0; p < kPairs; p++) g[p] = SF ? (hit[p] ? g[p] * y[p] : 0.0) : g[p] * y[p];
   side_by_side();
+}
+
+template <bool SF>
+__device__ __forceinline__ void pairs_force(const Replica& R, const double* dx, const double* dy, const double* dz,
+                                            PairAcc& a) {
+  double g[kPairs];
+  pairs_factor<SF>(R, dx, dy, dz, g);
 #pragma unroll
   for (int p = 0; p < kPairs; p++) {
     a.ax = __builtin_fma(dx[p], g[p], a.ax);
@@ -1684,15 +1698,20 @@ __device__ __forceinline__ void pairs_force(const Replica& R, const double* dx, 
 // f += (float)d fscal in FP32 over the eight entries of one list octet; the
 // caller adds each octet's f to the FP64 sum (pads add exactly 0).
 template <bool SF>
-__device__ __forceinline__ void pair_force_f32(const Replica& R, double dx, double dy, double dz, double r2,
-                                               float& fx, float& fy, float& fz) {
+__device__ __forceinline__ float pair_factor_f32(const Replica& R, double r2) {
   const bool hit = r2 < R.rc2;
   const float q = (float)r2;
   const float inv2 = rcp_rn_f32(q);
   const float s6 = inv2 * inv2 * inv2;
   float g = s6 * __builtin_fmaf(s6, 2.0f, -1.0f);
   if (SF) g = __builtin_fmaf(-__builtin_sqrtf(q), (float)R.force_shift24, g);
-  const float fscal = hit ? g * inv2 : 0.0f;
+  return hit ? g * inv2 : 0.0f;
+}
+
+template <bool SF>
+__device__ __forceinline__ void pair_force_f32(const Replica& R, double dx, double dy, double dz, double r2,
+                                               float& fx, float& fy, float& fz) {
+  const float fscal = pair_factor_f32<SF>(R, r2);
   fx = __builtin_fmaf((float)dx, fscal, fx);
   fy = __builtin_fmaf((float)dy, fscal, fy);
   fz = __builtin_fmaf((float)dz, fscal, fz);
@@ -1878,74 +1897,64 @@ __device__ __forceinline__ PairAcc interactions(const Buffers& B, const Replica&
 // `moved`, when the replica's lists were rebuilt on this step: the state in the
 // new order is where the list build left it (positions in xb, the rest in the
 // second set), and goes to the main set from here.
-template <int PREC, bool SF, class L>
-__device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
-                                           uint32_t gb, bool staged, int kick, bool moved) {
-  const uint32_t H = S.hoff[home_cells(g)];
-  const double *X = moved ? B.xb : B.x, *Y = moved ? B.yb : B.y, *Z = moved ? B.zb : B.z;
-  unsigned long long far = 0ull;
-  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
-    const Home at = home_atom(g, S, h);
-    const uint32_t i = at.slot;
-    double xi, yi, zi;
-    staged_pos(R, S, staged, at.e, X, Y, Z, xi, yi, zi);
-    double* const A[3] = {B.ax, B.ay, B.az};
-    double* const V[3] = {B.vx, B.vy, B.vz};
-    const double* const V2[3] = {B.vx2, B.vy2, B.vz2};
-    const double* const A2[3] = {B.ax2, B.ay2, B.az2};
-    const double* const XB[3] = {B.xb, B.yb, B.zb};
-    // The atom's own v and a, loaded before its pairs so that the loads are
-    // in flight while they are summed (the 512-replica batch +3.3%, FCC-1M
-    // +0.9%) -- in the plain (truncated and shifted) forms; the
-    // shifted-force pair loops leave no room for them within 128 VGPRs.
-    constexpr bool kEarly = !SF;
-    double vo[3], ao[3] = {0.0, 0.0, 0.0};
-    auto own_state = [&] {
+struct Own {  // an atom's own state before its kick
+  double v[3], a[3];
+  __device__ __forceinline__ void load(const Buffers& B, uint32_t i, int kick, bool moved) {
+    const double* const V[3] = {moved ? B.vx2 : B.vx, moved ? B.vy2 : B.vy, moved ? B.vz2 : B.vz};
+    const double* const A[3] = {moved ? B.ax2 : B.ax, moved ? B.ay2 : B.ay, moved ? B.az2 : B.az};
 #pragma unroll
-      for (int k = 0; k < 3; k++) vo[k] = (moved ? V2[k] : V[k])[i];
-      if (kick == 2) {
+    for (int k = 0; k < 3; k++) v[k] = V[k][i];
 #pragma unroll
-        for (int k = 0; k < 3; k++) ao[k] = (moved ? A2[k] : A[k])[i];
-      }
-    };
-    if constexpr (kEarly) own_state();
-    const PairAcc G = interactions<PREC, SF, false>(B, R, S, staged, X, Y, Z, i, xi, yi, zi);
-    if constexpr (!kEarly) own_state();
-    const double a[3] = {-24.0 * G.ax, -24.0 * G.ay, -24.0 * G.az};
-    const double xo[3] = {xi, yi, zi};
-    if (moved) {
-      double* const X1[3] = {B.x, B.y, B.z};
+    for (int k = 0; k < 3; k++) a[k] = kick == 2 ? A[k][i] : 0.0;
+  }
+};
+
+// Everything of atom i after its pair sums (at x[3], its position at the last
+// list build by built(k)); `far` takes its moved^2 in the drift-ahead form.
+template <class F>
+__device__ __forceinline__ void finish_atom(const Buffers& B, const Replica& R, int kick, bool moved, uint32_t i,
+                                            const double x[3], const Own& o, const PairAcc& sum, F&& built,
+                                            unsigned long long& far) {
+  double* const A[3] = {B.ax, B.ay, B.az};
+  double* const V[3] = {B.vx, B.vy, B.vz};
+  const double a[3] = {-24.0 * sum.ax, -24.0 * sum.ay, -24.0 * sum.az};
+  if (moved) {
+    double* const X1[3] = {B.x, B.y, B.z};
 #pragma unroll
-      for (int k = 0; k < 3; k++) X1[k][i] = xo[k];
-      B.orig[i] = B.orig2[i];
-      if (kick == 0) {
+    for (int k = 0; k < 3; k++) X1[k][i] = x[k];
+    B.orig[i] = B.orig2[i];
+    if (kick == 0) {
 #pragma unroll
-        for (int k = 0; k < 3; k++) V[k][i] = vo[k];
-      }
-    }
-    if (kick == 2) {
-      double* const X2[3] = {B.x2, B.y2, B.z2};
-      double d[3];
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        const double half = __builtin_fma(ao[k], R.half_dt, vo[k]);  // the drift's half step
-        const double v = __builtin_fma(a[k], R.half_dt, half);
-        A[k][i] = a[k];
-        V[k][i] = v;
-        const double x = __builtin_fma(__builtin_fma(a[k], R.half_dt, v), R.dt, xo[k]);
-        X2[k][i] = x;
-        d[k] = x - XB[k][i];
-      }
-      const unsigned long long m = (unsigned long long)__double_as_longlong(dist2(d[0], d[1], d[2]));
-      far = m > far ? m : far;
-    } else {
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        A[k][i] = a[k];
-        if (kick) V[k][i] = __builtin_fma(a[k], R.half_dt, vo[k]);
-      }
+      for (int k = 0; k < 3; k++) V[k][i] = o.v[k];
     }
   }
+  if (kick == 2) {
+    double* const X2[3] = {B.x2, B.y2, B.z2};
+    double d[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      const double half = __builtin_fma(o.a[k], R.half_dt, o.v[k]);  // the drift's half step
+      const double v = __builtin_fma(a[k], R.half_dt, half);
+      A[k][i] = a[k];
+      V[k][i] = v;
+      const double xn = __builtin_fma(__builtin_fma(a[k], R.half_dt, v), R.dt, x[k]);
+      X2[k][i] = xn;
+      d[k] = xn - built(k);
+    }
+    const unsigned long long m = (unsigned long long)__double_as_longlong(dist2(d[0], d[1], d[2]));
+    far = m > far ? m : far;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      A[k][i] = a[k];
+      if (kick) V[k][i] = __builtin_fma(a[k], R.half_dt, o.v[k]);
+    }
+  }
+}
+
+// The workgroup's maxima after its atoms.
+__device__ __forceinline__ void finish_brick(const Buffers& B, const Brick& g, uint32_t gb, int kick,
+                                             unsigned long long far) {
   if (kick == 2) {
     far = wave_max_u64(far);
     if ((threadIdx.x & 63u) == 0 && far != 0ull)
@@ -1955,6 +1964,32 @@ __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, c
     if (threadIdx.x == 0)
       for (uint32_t k = gb; k < B.n_replicas * kAheadSlots; k += B.n_bricks) B.amax[k] = 0ull;
   }
+}
+
+template <int PREC, bool SF, class L>
+__device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
+                                           uint32_t gb, bool staged, int kick, bool moved) {
+  const uint32_t H = S.hoff[home_cells(g)];
+  const double *X = moved ? B.xb : B.x, *Y = moved ? B.yb : B.y, *Z = moved ? B.zb : B.z;
+  unsigned long long far = 0ull;
+  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
+    const Home at = home_atom(g, S, h);
+    const uint32_t i = at.slot;
+    double x[3];
+    staged_pos(R, S, staged, at.e, X, Y, Z, x[0], x[1], x[2]);
+    const double* const XB[3] = {B.xb, B.yb, B.zb};
+    // The atom's own v and a, loaded before its pairs so that the loads are
+    // in flight while they are summed (the 512-replica batch +3.3%, FCC-1M
+    // +0.9%) -- in the plain (truncated and shifted) forms; the
+    // shifted-force pair loops leave no room for them within 128 VGPRs.
+    constexpr bool kEarly = !SF;
+    Own o;
+    if constexpr (kEarly) o.load(B, i, kick, moved);
+    const PairAcc sum = interactions<PREC, SF, false>(B, R, S, staged, X, Y, Z, i, x[0], x[1], x[2]);
+    if constexpr (!kEarly) o.load(B, i, kick, moved);
+    finish_atom(B, R, kick, moved, i, x, o, sum, [&](int k) { return XB[k][i]; }, far);
+  }
+  finish_brick(B, g, gb, kick, far);
 }
 
 // One workgroup per brick, leaving bricks that are cut (see k_build) to the
@@ -1984,6 +2019,226 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
       force_part<PREC, SF>(B, R, S, g, gb, staged, kick, moved);
     });
   }
+}
+
+// A brick of one or two waves of home atoms leaves the rest of its workgroup
+// idle, and its pairs run one after the other in those waves. Its G waves per
+// block of 64 home atoms (a crew) share them instead: each takes an octet of
+// every atom's list and leaves the pair factors in LDS, past the staged atoms,
+// then the crew's first waves add the octets up in list order, an axis each:
+// the same operations in the same order, only the factors are found side by
+// side. What is left is the chain of loads (~0.7 us each) in front of the first
+// pair, so the home atoms' counts, first octets and own state are loaded beside
+// the positions that are staged. us/step without / with crews: 1000 atoms 18.9 /
+// 17.2, 16,384 with the heat current every second step 65.8 / 57 a sample, a
+// driven 10 x 10 x 40 box 42.7 / 39.4. Bricks of more blocks gain nothing: 50,653
+// atoms (200 a brick, crews of two) 36.9 / 43.6 us/step, so the planner's bricks
+// take crews up to kCrewAtoms atoms.
+constexpr uint32_t kCrewWaves = Dense::kThreads / 64;
+constexpr uint32_t kCrewOctet = 512;  // factors of one wave's octet: 8 entries x 64 atoms
+
+// The most staged atoms that leave room for every wave's octet, spread over
+// the ends of the three position arrays.
+constexpr uint32_t kCrewStaged = Dense::kListPad - (kCrewWaves + 2u) / 3u * kCrewOctet;
+
+// Where wave w leaves its factors.
+__device__ __forceinline__ double* crew_octet(Stage<Dense>& S, uint32_t w) {
+  return S.x + (w % 3u) * (Dense::kStageMax + 64) + (Dense::kListPad - (w / 3u + 1u) * kCrewOctet);
+}
+
+// This wave's part in the crews of its brick: member `member` of the G waves of
+// block `block` of W (G = 0: the brick takes no crews).
+struct Crew {
+  const Buffers& B;
+  const Replica& R;
+  const Brick& g;
+  Stage<Dense>& S;
+  uint32_t* most;  // by wave: the longest list, in octets
+  int kick;
+  bool moved;
+  uint32_t G, W, block, member;
+  bool on;  // the lane stands for home atom i of its wave's block
+  uint32_t i, e, count;
+  const uint16_t* lst;
+  u32x4 mine;
+  Own o;
+  double xb[3];
+
+  __device__ __forceinline__ void cells_known() {
+    const uint32_t H = S.hoff[home_cells(g)];
+    W = (H + 63u) / 64u;
+    G = W == 0u || 2u * W > kCrewWaves || S.total > kCrewStaged ? 0u : kCrewWaves / W >= 8u ? 8u : kCrewWaves / W >= 4u ? 4u : 2u;
+    if (G == 0u) return;
+    const uint32_t wave = uniform(threadIdx.x >> 6);
+    block = wave % W;
+    member = wave / W;
+    const uint32_t h = 64u * block + (threadIdx.x & 63u);
+    on = h < H && member < G;
+    const Home at = home_atom(g, S, on ? h : 0u);
+    i = at.slot;
+    e = at.e;
+    count = B.nbr_count[i];
+    lst = B.nbr + list_base(R, i - R.atom_off);
+    // the count is not waited for: any octet of the list's own room
+    mine = load_octet(lst, member, list_octets(R.capacity) - 1u);
+    if (member == 0u) {
+      o.load(B, i, kick, moved);
+      xb[0] = B.xb[i];
+      xb[1] = B.yb[i];
+      xb[2] = B.zb[i];
+    }
+  }
+  __device__ __forceinline__ void loads_done() {
+    if (G == 0u) return;
+    const uint32_t longest = (uint32_t)wave_max_u64(on ? (count + 7u) / 8u : 0u);
+    if ((threadIdx.x & 63u) == 0u) most[threadIdx.x >> 6] = longest;
+  }
+};
+
+// The pair sums of a brick's atoms by its crews of G waves; every wave of the
+// workgroup calls it. Member 0 of each crew returns with its atoms' sums.
+template <int PREC, bool SF, int G>
+__device__ __forceinline__ PairAcc interactions_crew(const Replica& R, Stage<Dense>& S, const Crew& c, double xi,
+                                                     double yi, double zi) {
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t no = c.on ? (c.count + 7u) / 8u : 0u;
+  const uint32_t last = no > 0u ? no - 1u : 0u;
+  uint32_t octets = 0u;
+#pragma unroll
+  for (uint32_t w = 0; w < kCrewWaves; w++) octets = max(octets, c.most[w]);
+  const bool adds = c.member < (G < 3 ? (uint32_t)G : 3u);
+  const double* const C = c.member == 0u ? S.x : c.member == 1u ? S.y : S.z;  // the axis this wave adds up
+  const double own = c.member == 0u ? xi : c.member == 1u ? yi : zi;
+  double* const left = crew_octet(S, wave);
+  u32x4 mine = c.mine;
+  double f = 0.0, fz = 0.0;
+  for (uint32_t first = 0; first < octets; first += G) {
+    u32x4 all[G];
+    if (adds) {
+#pragma unroll
+      for (uint32_t j = 0; j < (uint32_t)G; j++) all[j] = load_octet(c.lst, first + j, last);
+    }
+    double g[8];
+    const bool has = first + c.member < no;
+    if (has) {
+      const uint32_t w[4] = {mine.x, mine.y, mine.z, mine.w};
+      double dx[8], dy[8], dz[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint32_t off = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;  // 8 e
+        dx[k] = *(const double*)((const char*)S.x + off);
+        dy[k] = *(const double*)((const char*)S.y + off);
+        dz[k] = *(const double*)((const char*)S.z + off);
+      }
+      side_by_side();
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        dx[k] -= xi;
+        dy[k] -= yi;
+        dz[k] -= zi;
+      }
+      if constexpr (PREC == 0) {
+#pragma unroll
+        for (int k = 0; k < 8; k += kPairs) pairs_factor<SF>(R, dx + k, dy + k, dz + k, g + k);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; k++) g[k] = (double)pair_factor_f32<SF>(R, dist2(dx[k], dy[k], dz[k]));
+      }
+    }
+    mine = load_octet(c.lst, first + G + c.member, last);
+    if (first) __syncthreads();  // the octets before have been added up
+    if (has) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) left[64 * k + lane] = g[k];
+    }
+    __syncthreads();
+    if (adds) {
+      // octet j's coordinates and factors come from LDS while the one before
+      // is added up
+      constexpr int kAxes = G < 3 ? 2 : 1;
+      double d[2][kAxes][8], p[2][8];
+      auto fetch = [&](uint32_t j) {
+        const u32x4 o = first + j < no ? all[j] : u32x4{0u, 0u, 0u, 0u};
+        const uint32_t w[4] = {o.x, o.y, o.z, o.w};
+        const double* const q = crew_octet(S, c.block + j * c.W) + lane;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          const uint32_t off = (w[k >> 1] >> ((k & 1) * 16)) & 0xffffu;
+          d[j & 1u][0][k] = *(const double*)((const char*)C + off);
+          if (kAxes == 2) d[j & 1u][kAxes - 1][k] = *(const double*)((const char*)S.z + off);
+          p[j & 1u][k] = q[64 * k];
+        }
+      };
+      auto add = [&](const double* x, const double* q, double at, double& sum) {
+        if constexpr (PREC == 0) {
+#pragma unroll
+          for (int k = 0; k < 8; k++) sum = __builtin_fma(x[k] - at, q[k], sum);
+        } else {
+          float part = 0.0f;
+#pragma unroll
+          for (int k = 0; k < 8; k++) part = __builtin_fmaf((float)(x[k] - at), (float)q[k], part);
+          sum += (double)part;
+        }
+      };
+      fetch(0u);
+#pragma unroll
+      for (uint32_t j = 0; j < (uint32_t)G; j++) {
+        if (j + 1u < (uint32_t)G) fetch(j + 1u);
+        side_by_side();
+        if (first + j < no) {
+          add(d[j & 1u][0], p[j & 1u], own, f);
+          if (kAxes == 2) add(d[j & 1u][kAxes - 1], p[j & 1u], zi, fz);
+        }
+        side_by_side();
+      }
+    }
+  }
+  __syncthreads();
+  if (adds && c.member != 0u) left[lane] = f;
+  __syncthreads();
+  PairAcc a = {0.0, 0.0, 0.0, 0.0, 0.0, 0u, 0u};
+  if (c.member == 0u) {
+    a.ax = f;
+    a.ay = crew_octet(S, c.block + c.W)[lane];
+    a.az = G < 3 ? fz : crew_octet(S, c.block + 2u * c.W)[lane];
+  }
+  return a;
+}
+
+template <int PREC, bool SF, int G>
+__device__ __forceinline__ void force_crew(const Buffers& B, const Replica& R, Stage<Dense>& S, const Crew& c,
+                                           uint32_t gb) {
+  const double x[3] = {S.x[c.e], S.y[c.e], S.z[c.e]};
+  const PairAcc sum = interactions_crew<PREC, SF, G>(R, S, c, x[0], x[1], x[2]);
+  unsigned long long far = 0ull;
+  if (c.on && c.member == 0u)
+    finish_atom(B, R, c.kick, c.moved, c.i, x, c.o, sum, [&](int k) { return c.xb[k]; }, far);
+  finish_brick(B, c.g, gb, c.kick, far);
+}
+
+// k_force of dense bricks that are small enough for crews; a brick that is not
+// goes as there. One workgroup a CU, so up to 256 VGPRs: held to 128 it spills
+// ~140 of them (1000 atoms 25 us/step).
+template <int PREC, bool SF>
+__global__ void __launch_bounds__(Dense::kThreads, 2) k_force_crews(Buffers B, int kick) {
+  __shared__ Stage<Dense> S;
+  __shared__ uint32_t most[kCrewWaves];
+  const uint32_t gb = dealt_index(blockIdx.x);
+  if (gb >= layout_end<Dense>(B)) return;
+  const Brick g = B.bricks[gb];
+  const Replica R = B.rep[g.rep];
+  const bool moved = B.ctl[g.rep].rebuild != 0u;
+  Crew c = {B, R, g, S, most, kick, moved};
+  const bool staged = stage_brick(B, R, g, moved ? B.xb : B.x, moved ? B.yb : B.y, moved ? B.zb : B.z, S, nullptr, c);
+  if (!staged && home_cells(g) > 1u && B.parts_on) return;  // cut into parts
+  if (c.G == 8u)
+    force_crew<PREC, SF, 8>(B, R, S, c, gb);
+  else if (c.G == 4u)
+    force_crew<PREC, SF, 4>(B, R, S, c, gb);
+  else if (c.G == 2u)
+    force_crew<PREC, SF, 2>(B, R, S, c, gb);
+  else
+    force_part<PREC, SF>(B, R, S, g, gb, staged, kick, moved);
 }
 
 // ---------------------------------------------------------------------------
@@ -3040,7 +3295,9 @@ hipError_t force_launches(const Buffers& B, int k, hipStream_t s, const Side* si
   const dim3 gp = parts_grid(B);
   hipError_t e = hipSuccess;
   const hipStream_t ss = fork_side(B, s, side, e);
-  if (layout_count<Dense>(B))
+  if (layout_count<Dense>(B) && B.crews)
+    hipLaunchKernelGGL((k_force_crews<PREC, SF>), brick_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, k);
+  else if (layout_count<Dense>(B))
     hipLaunchKernelGGL((k_force<Dense, PREC, SF, false>), brick_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, k);
   if (layout_count<Sparse>(B))
     hipLaunchKernelGGL((k_force<Sparse, PREC, SF, false>), brick_grid<Sparse>(B), dim3(Sparse::kThreads), 0, ss, B, k);

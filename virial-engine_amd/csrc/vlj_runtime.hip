@@ -54,6 +54,9 @@ constexpr double kSpreadAtoms = 64.0;
 // 15,600 atoms ran 1% slower (12% at 244).
 constexpr double kSpreadMost = 384.0;
 constexpr double kNoSpread = 1e300;
+// Bricks planned to own at most this many atoms take crews (k_force_crews):
+// two blocks of a wave, four waves to each.
+constexpr double kCrewAtoms = 128.0;
 // Atoms per staged cell from which a layer keeps the dense layout however few
 // its bricks stage: a small brick of a liquid fits the sparse layout's 1024
 // atoms, but that layout's build gives each home atom to one lane, which tests
@@ -734,6 +737,7 @@ int upload_table(vlj_sim* s) {
   }
   B.n_bricks = (uint32_t)nb;
   B.n_dense = s->n_dense;
+  B.crews = plan_spread(s) <= kCrewAtoms;
   HIP_TRY(s, hipMemcpy((void*)B.bricks, s->bricks.data(), nb * sizeof(Brick), hipMemcpyHostToDevice));
   HIP_TRY(s, hipMemset(B.cut, 0, std::max<size_t>(nb, 1) * 4));
   HIP_TRY(s, hipMemset(B.cut_groups, 0, std::max<size_t>(ng, 1) * 4));
@@ -1107,6 +1111,7 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   B.bricks = gb;
   B.n_bricks = (uint32_t)s->bricks.size();
   B.n_dense = s->n_dense;
+  B.crews = plan_spread(s) <= kCrewAtoms;
   B.parts_on = g_plan.parts >= 0 ? (uint32_t)g_plan.parts : (any_overflow(s, occs) ? 1u : 0u);
   B.n_atom_blocks = (uint32_t)s->atom_blocks.size();
   B.n_scan_blocks = (uint32_t)s->scan_blocks.size();
@@ -2678,6 +2683,7 @@ int vlj_load(const char* path, vlj_sim** out) {
   s->bricks = bricks;
   s->n_dense = h.n_dense;
   B.n_dense = h.n_dense;
+  B.crews = plan_spread(s) <= kCrewAtoms;
   B.parts_on = std::any_of(a.cut.begin(), a.cut.end(), [](uint32_t np) { return np != 0u; }) ? 1u : 0u;
   s->rep_bricks.assign(R, 0u);
   for (const Brick& g : bricks) s->rep_bricks[g.rep]++;
