@@ -70,6 +70,14 @@ __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
   return v;
 }
 
+// A value that is the same in every lane, as a scalar.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// A lane's value read from lane `l` (the same in every lane), as a scalar.
+__device__ __forceinline__ uint32_t readlane_u32(uint32_t v, uint32_t l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
+}
+
 // Reads a word another workgroup wrote, past this CU's L1.
 __device__ __forceinline__ uint32_t load_agent(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -659,6 +667,13 @@ __global__ void __launch_bounds__(kBlock) k_scatter(Buffers B) {
 // cells of a dense replica (a wave per cell) or kSortCellsSparse of a dilute
 // one: there a thread ranks a cell of at most kSmallCell atoms on its own,
 // and the waves take the larger cells of the block in turn.
+// The cells a wave ranks are loaded kSortFlight at a time, and their entries go
+// round by readlane instead of through LDS: with one cell in flight a wave waited
+// for each, 64 times where a liquid lies in a dilute replica's block (a rebuild of
+// a 524,309-atom slab 84 us in this kernel; that slab's step 201 -> 196 us, a
+// batch of 96 replicas 304 -> 301).
+constexpr uint32_t kSortFlight = 8;
+
 __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
   if (*B.rebuilding == 0u) return;  // no replica rebuilds this step
   const uint32_t sb = dealt_index(blockIdx.x);
@@ -696,21 +711,31 @@ __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
     }
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const uint32_t nb = n_big;
-  for (uint32_t k = threadIdx.x >> 6; k < nb; k += kBlock / 64) {
-    const uint32_t start = big_start[k], n = big_n[k];
-    if (n <= 64u) {
-      uint32_t e = lane < (int)n ? B.unsorted[start + lane] : 0xffffffffu;
-      uint32_t rank = 0;
-      for (uint32_t m = 0; m < n; m++) rank += (__shfl(e, (int)m, 64) < e) ? 1u : 0u;
-      if (lane < (int)n) B.sorted[start + rank] = e;
-    } else {
-      for (uint32_t j = (uint32_t)lane; j < n; j += 64u) {
-        uint32_t e = B.unsorted[start + j];
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t nb = n_big, waves = kBlock / 64;
+  for (uint32_t k0 = uniform(threadIdx.x >> 6); k0 < nb; k0 += waves * kSortFlight) {
+    uint32_t e[kSortFlight];
+#pragma unroll
+    for (uint32_t j = 0; j < kSortFlight; j++) {
+      const uint32_t k = k0 + j * waves;
+      e[j] = k < nb && lane < big_n[k] ? B.unsorted[big_start[k] + lane] : 0xffffffffu;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kSortFlight; j++) {
+      const uint32_t k = k0 + j * waves;
+      if (k >= nb) break;
+      const uint32_t start = uniform(big_start[k]), n = uniform(big_n[k]);
+      if (n <= 64u) {
         uint32_t rank = 0;
-        for (uint32_t m = 0; m < n; m++) rank += (B.unsorted[start + m] < e) ? 1u : 0u;
-        B.sorted[start + rank] = e;
+        for (uint32_t m = 0; m < n; m++) rank += readlane_u32(e[j], m) < e[j] ? 1u : 0u;
+        if (lane < n) B.sorted[start + rank] = e[j];
+      } else {
+        for (uint32_t q = lane; q < n; q += 64u) {
+          const uint32_t v = B.unsorted[start + q];
+          uint32_t rank = 0;
+          for (uint32_t m = 0; m < n; m++) rank += (B.unsorted[start + m] < v) ? 1u : 0u;
+          B.sorted[start + rank] = v;
+        }
       }
     }
   }
@@ -802,7 +827,7 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 // by DPP moves, home atoms numbered in the same pass as the staged ones, no
 // integer division a cell. us/step before (shuffles, a third scan by one wave,
 // 8 divisions a cell) / with: 1000 atoms 20.1 / 19.2, 50,653 36.9 / 36.0, FCC-1M
-// 196 / 191 (FP32 190 / 184), the 16-replica batch 314 / 306.
+// 196 / 191 (FP32 190 / 184), a batch of 96 replicas 314 / 306.
 struct NoCrew {
   __device__ __forceinline__ void cells_known() {}
   __device__ __forceinline__ void loads_done() {}
@@ -1015,8 +1040,6 @@ __device__ __forceinline__ void staged_pos(const Replica& R, const Stage<L>& S, 
   }
 }
 
-// A value that is the same in every lane, as a scalar.
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 
 // A brick whose neighbourhood holds more than kStageMax atoms (the density
 // rose since the bricks were planned) is cut into parts: each of its cell
@@ -1176,10 +1199,6 @@ __device__ __forceinline__ uint32_t lane_rank(unsigned long long mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// A lane's value read from lane `l` (the same in every lane), as a scalar.
-__device__ __forceinline__ uint32_t readlane_u32(uint32_t v, uint32_t l) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
-}
 
 // Atoms of a home cell per work item of the list build, and chunks of 64
 // candidates a wave holds in registers at once.
@@ -1618,7 +1637,7 @@ __device__ __forceinline__ void pair_accumulate(const Replica& R, double dx, dou
 // to itself, waits for each LDS gather where it is used and runs one pair after
 // the other, so that a wave stands idle at every step of both. Measured
 // (MI355X, us/step, before / with 2 / with 4 / with 8 pairs): 1000 atoms 22.4 /
-// 20.1 / 20.1 / 21.2, FCC-1M 198 / 195 / 197 / 212, the 16-replica batch 318 /
+// 20.1 / 20.1 / 21.2, FCC-1M 198 / 195 / 197 / 212, a batch of 96 replicas 318 /
 // 312 / 313 / -: 8 pairs do not fit beside the octets in flight at 4 waves per
 // SIMD. 4 FP32 pairs side by side measured the same as the plain loop
 // (FCC-1M 192 us/step either way), which stays.
@@ -2030,7 +2049,7 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
 // side. What is left is the chain of loads (~0.7 us each) in front of the first
 // pair, so the home atoms' counts, first octets and own state are loaded beside
 // the positions that are staged. us/step without / with crews: 1000 atoms 18.9 /
-// 17.2, 16,384 with the heat current every second step 65.8 / 57 a sample, a
+// 17.2, 3458 with the heat current every second step 65.8 / 57 a sample, a
 // driven 10 x 10 x 40 box 42.7 / 39.4. Bricks of more blocks gain nothing: 50,653
 // atoms (200 a brick, crews of two) 36.9 / 43.6 us/step, so the planner's bricks
 // take crews up to kCrewAtoms atoms.

@@ -25,9 +25,9 @@ constexpr int kRing = 3;         // read-back slots (lennard_jones.rs:320)
 // Steps are captured in graphs of 2^k of them, k below kGraphs, each on its
 // first use: a call for few steps between two samples is one or two launches
 // (a graph launch takes ~10 us on the host and leaves a gap of several us).
-// 16,384 atoms, a heat-current sample every second step, us per sample with
+// 3458 atoms, a heat-current sample every second step, us per sample with
 // graphs of 1 and 16 only / these: 75.6 / 65.8; a profile sample every 20 steps,
-// 4096 atoms: 437 / 428.
+// 3377 atoms: 437 / 428.
 constexpr uint32_t kGraphs = 5;
 // Brick planner. Bricks are planned to stage at most kDefaultFill of the
 // LDS staging limit until the tuner has measured the candidates kTuneFills
