@@ -100,3 +100,22 @@ def test_heat_exchange_moves_energy_and_keeps_momentum(oracle, lj):
     for k in range(3):
         assert abs(after.momentum[k] - before.momentum[k]) < 1e-6 * after.count
     assert t[0] > t[6] + 0.04
+
+
+@pytest.mark.parametrize("n", [700, 1025, 8192, 8193])  # one workgroup's width, its last atom count, one atom past it
+def test_heat_exchange_of_any_size_is_bit_exact(oracle, lj, n):
+    side = (n / 0.8) ** (1.0 / 3.0)
+    hot, cold = (0.0, 0.2 * side), (0.5 * side, 0.7 * side)
+    pos, vel = oracle.lattice(n, side, 1.0, 9)
+    sim = lj.LennardJones((pos, vel), lj.Settings([side] * 3, 2.5, 0.002, skin=0.3, shifted_force=True))
+    ref = oracle.Sim(pos, vel, [side] * 3, cutoff=2.5, skin=0.3, dt=0.002, shifted_force=True)
+    sim.set_heat_exchange(lj.HeatExchange(hot, cold, 0.02))
+    ref.set_heat_exchange(hot, cold, 0.02)
+    for steps in (1, 30):
+        sim.run(steps)
+        ref.run(steps)
+        assert list(sim.measure_now().raw) == list(ref.measure().raw)
+        a = sim.read_particle_array()
+        rp, rv = ref.read_particles()
+        np.testing.assert_array_equal(a["pos"], rp)
+        np.testing.assert_array_equal(a["vel"], rv)

@@ -306,6 +306,70 @@ __device__ __forceinline__ int hex_slab(const Replica& R, double z) {
   return 2;
 }
 
+// Atom i's terms of its slab's sums, added to q.
+__device__ __forceinline__ void hex_terms(const Buffers& B, const Replica& R, uint32_t i, int slab,
+                                          long long q[kHexSums]) {
+  const double v[3] = {B.vx[i], B.vy[i], B.vz[i]};
+  const double f[3] = {B.ax[i], B.ay[i], B.az[i]};
+  long long t[9];
+  t[0] = 1;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    t[1 + k] = to_fixed(v[k], R.momentum_fixed);
+    t[6 + k] = to_fixed(f[k], R.momentum_fixed);
+  }
+  t[4] = to_fixed(dist2(v[0], v[1], v[2]), R.energy_fixed);
+  t[5] = to_fixed(__builtin_fma(f[2], v[2], __builtin_fma(f[1], v[1], f[0] * v[0])), R.energy_fixed);
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    q[k] += slab == 0 ? t[k] : 0;
+    q[9 + k] += slab == 1 ? t[k] : 0;
+  }
+}
+
+// A slab's scales from its nine sums q.
+__device__ __forceinline__ void hex_scales(const Replica& R, int slab, const long long* q, double* o) {
+  const double dt3 = R.dt * R.dt * R.dt;
+  const double m = (double)q[0];
+#pragma unroll
+  for (int k = 0; k < 9; k++) o[k] = 0.0;
+  if (!(m > 0.0)) return;
+  double pm[3], fm[3];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    pm[k] = (double)q[1 + k] / R.momentum_fixed;
+    fm[k] = (double)q[6 + k] / R.momentum_fixed;
+    o[k] = pm[k] / m;      // centre-of-mass velocity
+    o[3 + k] = fm[k] / m;  // mean force
+  }
+  const double v2 = (double)q[4] / R.energy_fixed;
+  const double fv = (double)q[5] / R.energy_fixed;
+  const double pp = __builtin_fma(pm[2], pm[2], __builtin_fma(pm[1], pm[1], pm[0] * pm[0]));
+  const double kinetic = 0.5 * v2 - 0.5 * pp / m;
+  const double energy = slab == 0 ? R.hex_energy : -R.hex_energy;
+  const double flux = energy / R.dt;
+  const double x = energy / kinetic;
+  o[6] = x / (1.0 + __builtin_sqrt(1.0 + x));
+  const double power = fv - __builtin_fma(fm[2], o[2], __builtin_fma(fm[1], o[1], fm[0] * o[0]));
+  o[7] = dt3 * flux / (2.0 * kinetic * kinetic) * (flux / 48.0 + power / 6.0);
+  o[8] = dt3 * flux / (12.0 * kinetic);
+}
+
+// Atom i of a slab with the scales o.
+__device__ __forceinline__ void hex_exchange(const Buffers& B, uint32_t i, const double* o) {
+  double* X[3] = {B.x, B.y, B.z};
+  double* V[3] = {B.vx, B.vy, B.vz};
+  const double* A[3] = {B.ax, B.ay, B.az};
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const double v = V[k][i];
+    const double rel = v - o[k];
+    const double shift = o[7] * rel - o[8] * (A[k][i] - o[3 + k]);
+    X[k][i] = X[k][i] - shift;
+    V[k][i] = __builtin_fma(rel, o[6], v);
+  }
+}
+
 __global__ void __launch_bounds__(kBlock) k_hex_sum(Buffers B) {
   const uint32_t b = dealt_index(blockIdx.x);
   if (b >= B.n_atom_blocks) return;
@@ -319,23 +383,7 @@ __global__ void __launch_bounds__(kBlock) k_hex_sum(Buffers B) {
   if (i < blk.end) {
     const int slab = hex_slab(R, B.z[i]);
     if (slab < 2) {
-      const double v[3] = {B.vx[i], B.vy[i], B.vz[i]};
-      const double f[3] = {B.ax[i], B.ay[i], B.az[i]};
-      const long long c = 1;
-      long long t[9];
-      t[0] = c;
-#pragma unroll
-      for (int k = 0; k < 3; k++) {
-        t[1 + k] = to_fixed(v[k], R.momentum_fixed);
-        t[6 + k] = to_fixed(f[k], R.momentum_fixed);
-      }
-      t[4] = to_fixed(dist2(v[0], v[1], v[2]), R.energy_fixed);
-      t[5] = to_fixed(__builtin_fma(f[2], v[2], __builtin_fma(f[1], v[1], f[0] * v[0])), R.energy_fixed);
-#pragma unroll
-      for (int k = 0; k < 9; k++) {
-        q[k] = slab == 0 ? t[k] : 0;
-        q[9 + k] = slab == 1 ? t[k] : 0;
-      }
+      hex_terms(B, R, i, slab, q);
     }
   }
   __shared__ long long part[kBlock / 64][kHexSums];
@@ -366,35 +414,8 @@ __global__ void __launch_bounds__(kBlock) k_hex_update(Buffers B) {
   }
   __syncthreads();
   if (threadIdx.x != 0) return;
-  double* out = B.hexstate + (size_t)r * kHexState;
-  const double dt3 = R.dt * R.dt * R.dt;
-  for (int slab = 0; slab < 2; slab++) {
-    const long long* q = sums + 9 * slab;
-    double* o = out + 9 * slab;
-    const double m = (double)q[0];
-#pragma unroll
-    for (int k = 0; k < 9; k++) o[k] = 0.0;
-    if (!(m > 0.0)) continue;
-    double pm[3], fm[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-      pm[k] = (double)q[1 + k] / R.momentum_fixed;
-      fm[k] = (double)q[6 + k] / R.momentum_fixed;
-      o[k] = pm[k] / m;      // centre-of-mass velocity
-      o[3 + k] = fm[k] / m;  // mean force
-    }
-    const double v2 = (double)q[4] / R.energy_fixed;
-    const double fv = (double)q[5] / R.energy_fixed;
-    const double pp = __builtin_fma(pm[2], pm[2], __builtin_fma(pm[1], pm[1], pm[0] * pm[0]));
-    const double kinetic = 0.5 * v2 - 0.5 * pp / m;
-    const double energy = slab == 0 ? R.hex_energy : -R.hex_energy;
-    const double flux = energy / R.dt;
-    const double x = energy / kinetic;
-    o[6] = x / (1.0 + __builtin_sqrt(1.0 + x));
-    const double power = fv - __builtin_fma(fm[2], o[2], __builtin_fma(fm[1], o[1], fm[0] * o[0]));
-    o[7] = dt3 * flux / (2.0 * kinetic * kinetic) * (flux / 48.0 + power / 6.0);
-    o[8] = dt3 * flux / (12.0 * kinetic);
-  }
+  for (int slab = 0; slab < 2; slab++)
+    hex_scales(R, slab, sums + 9 * slab, B.hexstate + (size_t)r * kHexState + 9 * slab);
 }
 
 __global__ void __launch_bounds__(kBlock) k_hex_apply(Buffers B) {
@@ -407,18 +428,60 @@ __global__ void __launch_bounds__(kBlock) k_hex_apply(Buffers B) {
   if (i >= blk.end) return;
   const int slab = hex_slab(R, B.z[i]);
   if (slab == 2) return;
-  const double* o = B.hexstate + (size_t)blk.rep * kHexState + 9 * slab;
-  double* X[3] = {B.x, B.y, B.z};
-  double* V[3] = {B.vx, B.vy, B.vz};
-  const double* A[3] = {B.ax, B.ay, B.az};
+  hex_exchange(B, i, B.hexstate + (size_t)blk.rep * kHexState + 9 * slab);
+}
+
+// The same of a replica of at most kChainAtoms atoms in one workgroup: three
+// launches cost such a replica more than what they do (3377 atoms, a driven 10 x
+// 10 x 40 box: 40.0 us/step with three launches, 35.2 with one). Larger ones keep
+// the three, which use every CU. A wave without an atom in a slab skips its sums.
+__global__ void __launch_bounds__(kChainThreads) k_hex_small(Buffers B) {
+  const uint32_t r = blockIdx.x, t = threadIdx.x;
+  const Replica R = B.rep[r];
+  if (!R.hex_on) return;
+  __shared__ long long part[kChainThreads / 64][kHexSums];
+  __shared__ long long sums[kHexSums];
+  __shared__ double scale[kHexSums];
+  const uint32_t end = R.atom_off + R.count;
+  double z[kChainPer];
+  int slab[kChainPer];
 #pragma unroll
-  for (int k = 0; k < 3; k++) {
-    const double v = V[k][i];
-    const double rel = v - o[k];
-    const double shift = o[7] * rel - o[8] * (A[k][i] - o[3 + k]);
-    X[k][i] = X[k][i] - shift;
-    V[k][i] = __builtin_fma(rel, o[6], v);
+  for (uint32_t k = 0; k < kChainPer; k++) {
+    const uint32_t i = R.atom_off + t + k * kChainThreads;
+    z[k] = i < end ? B.z[i] : 0.0;
   }
+  long long q[kHexSums];
+#pragma unroll
+  for (uint32_t k = 0; k < kHexSums; k++) q[k] = 0;
+  bool any = false;
+#pragma unroll
+  for (uint32_t k = 0; k < kChainPer; k++) {
+    const uint32_t i = R.atom_off + t + k * kChainThreads;
+    slab[k] = i < end ? hex_slab(R, z[k]) : 2;
+    if (slab[k] < 2) {
+      hex_terms(B, R, i, slab[k], q);
+      any = true;
+    }
+  }
+  const bool wave_any = __builtin_amdgcn_ballot_w64(any) != 0ull;
+#pragma unroll
+  for (uint32_t k = 0; k < kHexSums; k++) {
+    const long long w = wave_any ? wave_sum_i64(q[k]) : 0;
+    if ((t & 63u) == 0) part[t >> 6][k] = w;
+  }
+  __syncthreads();
+  if (t < kHexSums) {
+    long long x = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kChainThreads / 64; w++) x += part[w][t];
+    sums[t] = x;
+  }
+  __syncthreads();
+  if (t < 2u) hex_scales(R, (int)t, sums + 9 * t, scale + 9 * t);
+  __syncthreads();
+#pragma unroll
+  for (uint32_t k = 0; k < kChainPer; k++)
+    if (slab[k] < 2) hex_exchange(B, R.atom_off + t + k * kChainThreads, scale + 9 * slab[k]);
 }
 
 // ---------------------------------------------------------------------------
@@ -3196,6 +3259,10 @@ hipError_t launch_nh_half(const Buffers& B, bool scale, hipStream_t s) {
 
 hipError_t launch_heat_exchange(const Buffers& B, hipStream_t s) {
   if (!B.n_atom_blocks) return hipSuccess;
+  if (B.chain) {
+    hipLaunchKernelGGL(k_hex_small, decide_grid(B), dim3(kChainThreads), 0, s, B);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(k_hex_sum, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
   hipLaunchKernelGGL(k_hex_update, decide_grid(B), dim3(kBlock), 0, s, B);
   hipLaunchKernelGGL(k_hex_apply, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
