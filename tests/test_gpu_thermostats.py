@@ -88,3 +88,18 @@ def test_nose_hoover_samples_the_canonical_ensemble(oracle, lj):
     assert abs(ratio / canonical - 1) < 0.15
     assert abs(drift) < 1e-4
     assert end.list_overflow == 0
+
+
+@pytest.mark.parametrize("n", [65_536, 65_537])  # the most atoms whose kinetic energies each workgroup adds up, and past it
+def test_nose_hoover_of_many_blocks_is_bit_exact(oracle, lj, n):
+    side = (n / 0.3) ** (1.0 / 3.0)
+    pos, vel = oracle.lattice(n, side, 1.2, 5)
+    st = lj.Settings([side] * 3, 2.5, 0.002, thermostat=lj.NoseHoover(0.9, 0.2), shifted_force=True)
+    sim = lj.LennardJones((pos, vel), st)
+    ref = oracle.Sim(pos, vel, [side] * 3, dt=0.002, shifted_force=True, thermostat=2, temperature=0.9, period=0.2)
+    for steps in (1, 3):
+        sim.run(steps)
+        ref.run(steps)
+        m, r = sim.measure_now(), ref.measure()
+        assert list(m.raw) == list(r.raw)
+        assert m.thermostat_energy == r.thermostat_energy

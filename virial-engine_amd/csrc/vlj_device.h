@@ -155,6 +155,7 @@ struct Buffers {
   uint16_t* parts;            // per brick: kHomeCells packed parts
   uint32_t* cut_groups;       // per group of kCutGroup bricks: bricks cut
   uint32_t n_atom_blocks, n_scan_blocks, n_sort_blocks, n_bricks, n_replicas, n_dense;
+  uint32_t nh_inline;  // no replica has more than kInlineBlocks atom blocks: the kernels that scale find the scale
   uint32_t crews;  // the dense bricks are small: crews of waves share their atoms' pairs
   // 1: a brick whose neighbourhood outgrows LDS is cut into parts, which the
   // PARTS launches after each brick launch take; 0: no PARTS launches, and
@@ -162,6 +163,7 @@ struct Buffers {
   uint32_t parts_on;
   unsigned long long* bmax;   // per atom block: max moved^2 (FP64 bits)
   long long* kepart;          // per atom block: kinetic energy in fixed point (Nose-Hoover)
+  double* nh_in;  // per replica: friction and its integral before the Nose-Hoover half step
   long long* hexpart;         // per atom block: kHexSums heat-exchange sums
   double* hexstate;           // per replica: kHexState scales and corrections
   long long* hc;              // heat-current series of replica 0: 3 sums per sample
@@ -207,6 +209,12 @@ constexpr uint32_t kChainAtoms = 8192;
 constexpr uint32_t kChainCells = 8192;
 constexpr uint32_t kChainPer = kChainAtoms / kChainThreads;
 static_assert(kChainAtoms <= 0x10000u && kChainCells <= 0x10000u, "16-bit cells, ranks and places");
+
+// Nose-Hoover: up to this many atom blocks each workgroup that scales velocities
+// adds up its replica's kinetic energies itself (one load a thread) instead of
+// waiting for a launch between (eight slabs of 15,600 atoms 162 -> 157 us/step);
+// larger replicas would read thousands of them in every workgroup.
+constexpr uint32_t kInlineBlocks = kBlock;
 
 // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs on
 // XCD b % 8). Each table (atom blocks, sort blocks, bricks) is dealt to the

@@ -155,6 +155,42 @@ __global__ void __launch_bounds__(kBlock) k_decide(Buffers B, int advance) {
   }
 }
 
+// Friction, its integral and the velocity scale of replica r from its blocks'
+// kinetic energies and the friction before; every thread of the workgroup calls
+// it and gets the scale, and one workgroup (`keep`) leaves the new state.
+__device__ __forceinline__ double nh_update(const Buffers& B, const Replica& R, uint32_t r, bool keep) {
+  const double xi0 = B.nh_in[2u * r], eta0 = B.nh_in[2u * r + 1u];
+  long long t = 0;
+  for (uint32_t b = R.atom_block_off + threadIdx.x; b < R.atom_block_off + R.atom_blocks; b += kBlock)
+    t += B.kepart[b];
+  __shared__ long long part[kBlock / 64];
+  t = wave_sum_i64(t);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
+  __syncthreads();
+  long long raw = 0;
+#pragma unroll
+  for (int w = 0; w < kBlock / 64; w++) raw += part[w];
+  const double ke = (double)raw / R.energy_fixed;
+  const double quarter = 0.25 * R.dt;
+  const double xi = __builtin_fma((2.0 * ke - R.nh_gkt) / R.nh_q, quarter, xi0);
+  const double x = xi * R.half_dt;
+  const double sm1 = -x * (1.0 - x * (0.5 - x * (1.0 / 6.0 - x / 24.0)));
+  if (keep && threadIdx.x == 0) {
+    Control* c = B.ctl + r;
+    c->eta = __builtin_fma(xi, R.half_dt, eta0);
+    const double ke2 = __builtin_fma(ke, sm1 * (2.0 + sm1), ke);
+    c->xi = __builtin_fma((2.0 * ke2 - R.nh_gkt) / R.nh_q, quarter, xi);
+    c->sm1 = sm1;
+  }
+  return sm1;
+}
+
+// The scale for a workgroup of replica blk.rep: found here (B.nh_inline), or by
+// k_nh_update before. Every thread of the workgroup calls it.
+__device__ __forceinline__ double nh_scale(const Buffers& B, const Replica& R, const Range& blk) {
+  return B.nh_inline ? nh_update(B, R, blk.rep, blk.first == R.atom_off) : B.ctl[blk.rep].sm1;
+}
+
 // ---------------------------------------------------------------------------
 // Drift: v += a dt/2; x += v dt (or BAOAB); wrap; max moved^2 since build.
 // ---------------------------------------------------------------------------
@@ -173,6 +209,8 @@ __global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v, int to_
   const Replica R = B.rep[blk.rep];
   const uint32_t i = blk.first + threadIdx.x;
   unsigned long long moved = 0ull;
+  const bool nh = R.thermostat == 2u;
+  const double sm1 = nh ? nh_scale(B, R, blk) : 0.0;
   if (i < blk.end) {
     const bool baoab = LANGEVIN && R.thermostat == 1u;
     double n[3] = {0.0, 0.0, 0.0};
@@ -182,8 +220,6 @@ __global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v, int to_
     const double* A[3] = {B.ax, B.ay, B.az};
     const double* XB[3] = {B.xb, B.yb, B.zb};
     double d[3];
-    const bool nh = R.thermostat == 2u;
-    const double sm1 = nh ? B.ctl[blk.rep].sm1 : 0.0;
 #pragma unroll
     for (int k = 0; k < 3; k++) {
       double v0 = V[k][i];
@@ -246,6 +282,10 @@ __global__ void __launch_bounds__(kBlock) k_ke_sum(Buffers B) {
 #pragma unroll
     for (int w = 0; w < kBlock / 64; w++) t += part[w];
     B.kepart[b] = t;
+    if (blk.first == R.atom_off) {  // what the half step starts from
+      B.nh_in[2u * blk.rep] = B.ctl[blk.rep].xi;
+      B.nh_in[2u * blk.rep + 1u] = B.ctl[blk.rep].eta;
+    }
   }
 }
 
@@ -253,28 +293,7 @@ __global__ void __launch_bounds__(kBlock) k_nh_update(Buffers B) {
   const uint32_t r = blockIdx.x;
   const Replica R = B.rep[r];
   if (R.thermostat != 2u) return;
-  long long t = 0;
-  for (uint32_t b = R.atom_block_off + threadIdx.x; b < R.atom_block_off + R.atom_blocks; b += kBlock)
-    t += B.kepart[b];
-  __shared__ long long part[kBlock / 64];
-  t = wave_sum_i64(t);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    long long raw = 0;
-#pragma unroll
-    for (int w = 0; w < kBlock / 64; w++) raw += part[w];
-    Control* c = B.ctl + r;
-    const double ke = (double)raw / R.energy_fixed;
-    const double quarter = 0.25 * R.dt;
-    double xi = __builtin_fma((2.0 * ke - R.nh_gkt) / R.nh_q, quarter, c->xi);
-    const double x = xi * R.half_dt;
-    const double sm1 = -x * (1.0 - x * (0.5 - x * (1.0 / 6.0 - x / 24.0)));
-    c->eta = __builtin_fma(xi, R.half_dt, c->eta);
-    const double ke2 = __builtin_fma(ke, sm1 * (2.0 + sm1), ke);
-    c->xi = __builtin_fma((2.0 * ke2 - R.nh_gkt) / R.nh_q, quarter, xi);
-    c->sm1 = sm1;
-  }
+  (void)nh_update(B, R, r, true);
 }
 
 __global__ void __launch_bounds__(kBlock) k_nh_scale(Buffers B) {
@@ -283,9 +302,9 @@ __global__ void __launch_bounds__(kBlock) k_nh_scale(Buffers B) {
   const Range blk = B.atom_blocks[ab];
   const Replica R = B.rep[blk.rep];
   if (R.thermostat != 2u) return;
+  const double sm1 = nh_scale(B, R, blk);
   const uint32_t i = blk.first + threadIdx.x;
   if (i >= blk.end) return;
-  const double sm1 = B.ctl[blk.rep].sm1;
   B.vx[i] = __builtin_fma(B.vx[i], sm1, B.vx[i]);
   B.vy[i] = __builtin_fma(B.vy[i], sm1, B.vy[i]);
   B.vz[i] = __builtin_fma(B.vz[i], sm1, B.vz[i]);
@@ -3252,7 +3271,7 @@ hipError_t launch_drift(const Buffers& B, bool langevin, bool keep_v, bool decid
 hipError_t launch_nh_half(const Buffers& B, bool scale, hipStream_t s) {
   if (!B.n_atom_blocks) return hipSuccess;
   hipLaunchKernelGGL(k_ke_sum, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
-  hipLaunchKernelGGL(k_nh_update, decide_grid(B), dim3(kBlock), 0, s, B);
+  if (!B.nh_inline) hipLaunchKernelGGL(k_nh_update, decide_grid(B), dim3(kBlock), 0, s, B);
   if (scale) hipLaunchKernelGGL(k_nh_scale, grid1(dealt_grid(B.n_atom_blocks)), dim3(kBlock), 0, s, B);
   return hipGetLastError();
 }

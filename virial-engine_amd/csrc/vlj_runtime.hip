@@ -1080,6 +1080,7 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   A(&B.bmax, s->atom_blocks.size());
   A(&B.amax, 2 * replicas * kAheadSlots);
   A(&B.kepart, s->atom_blocks.size());
+  A(&B.nh_in, 2 * replicas);
   A(&B.hexpart, s->atom_blocks.size() * kHexSums);
   A(&B.hexstate, replicas * kHexState);
   double** d[] = {&B.x, &B.y, &B.z, &B.vx, &B.vy, &B.vz, &B.ax, &B.ay, &B.az,
@@ -1117,6 +1118,8 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   B.n_scan_blocks = (uint32_t)s->scan_blocks.size();
   B.n_sort_blocks = (uint32_t)s->sort_blocks.size();
   B.n_replicas = (uint32_t)replicas;
+  B.nh_inline = std::all_of(s->rep.begin(), s->rep.end(),
+                            [](const Replica& R) { return R.atom_blocks <= vlj::kInlineBlocks; });
   B.chain = std::all_of(s->rep.begin(), s->rep.end(), [](const Replica& R) {
     return R.count <= vlj::kChainAtoms && R.total_cells <= vlj::kChainCells;
   });
