@@ -139,3 +139,29 @@ def test_crews_against_the_oracle(oracle, lj, n, box, cutoff, shifted, precision
         assert list(sim.measure_now().raw) == list(ref.measure().raw)
         np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
         np.testing.assert_array_equal(sim.debug_state()[1], ref.state()[1])
+
+
+def test_shared_list_builds_against_the_oracle(oracle, lj):
+    # replicas of other sizes and densities on both layouts, each rebuilding on
+    # its own steps: several workgroups build each brick's lists
+    specs = []
+    for k, (n, rho, t) in enumerate([(1000, 0.8442, 0.7), (3001, 0.05, 1.5), (2048, 0.8, 1.2), (700, 0.3, 1.0),
+                                     (1, 0.02, 1.0)]):
+        side = (n / rho) ** (1.0 / 3.0)
+        parts = lj.lattice_array(n, max(side, 5.7), t, 41 + k)
+        specs.append((parts, lj.Settings([max(side, 5.7)] * 3, 2.5, 0.004, skin=0.3)))
+    sim = lj.Batch(specs)
+    for steps in (1, 30, 69):
+        sim.run(steps)
+    ms, allp = sim.measure_now(), sim.read_particle_array()
+    off = 0
+    for k, (parts, st) in enumerate(specs):
+        ref = oracle.Sim(np.ascontiguousarray(parts["pos"]), np.ascontiguousarray(parts["vel"]), list(st.box_size),
+                         cutoff=2.5, skin=0.3, dt=0.004)
+        ref.run(100)
+        r = ref.measure()
+        assert list(ms[k].raw) == list(r.raw) and ms[k].list_rebuilds == r.list_rebuilds, f"replica {k}"
+        pos, vel = ref.read_particles()
+        np.testing.assert_array_equal(allp["pos"][off:off + len(parts)], pos)
+        np.testing.assert_array_equal(allp["vel"][off:off + len(parts)], vel)
+        off += len(parts)

@@ -1300,10 +1300,11 @@ __device__ __forceinline__ uint32_t lane_rank(unsigned long long mask) {
 constexpr uint32_t kPiece = VLJ_BUILD_PIECE;
 constexpr int kGroup = VLJ_BUILD_GROUP;
 static_assert(kPiece >= 1 && kPiece <= 64, "a lane per home atom of a work item");
+constexpr uint32_t kLeast = 2;  // atoms of a piece, at least (1000 atoms: 16.6 us/step with 4, 16.3 with 2)
 static_assert(kListStride == 64, "entry pos of a list lies (pos / 8) KB + 2 (pos % 8) bytes from its base");
 
-// One workgroup per brick; its waves build the lists of one work item (a
-// piece of a home cell's atoms) at a time. A home cell's candidates are the
+// One or more workgroups per brick (share `share` of `shares`); their waves
+// build the lists of one work item (a piece of a home cell's atoms) at a time. A home cell's candidates are the
 // atoms of its 27 neighbour cells in list order: the nine runs (dz, dy) one
 // after the other, each run the three staged cells along x, which are
 // staged one after the other, so a run is one range of staged atoms. The
@@ -1326,10 +1327,10 @@ static_assert(kListStride == 64, "entry pos of a list lies (pos / 8) KB + 2 (pos
 template <class L>
 __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
                                             bool staged, const double* X, const double* Y, const double* Z,
-                                            const uint32_t* via) {
+                                            const uint32_t* via, uint32_t share, uint32_t shares) {
   const uint32_t cap = R.capacity;
   const uint32_t H = S.hoff[home_cells(g)];
-  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
+  for (uint32_t h = share * L::kThreads + threadIdx.x; h < H; h += shares * L::kThreads) {
     const Home a = home_atom(g, S, h);
     double xi, yi, zi;
     staged_pos(R, S, staged, a.e, X, Y, Z, xi, yi, zi, via);
@@ -1369,13 +1370,14 @@ __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, 
 template <class L>
 __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
                                            bool staged, bool relist, const double* X, const double* Y,
-                                           const double* Z, const uint32_t* via, uint32_t& next_item) {
+                                           const double* Z, const uint32_t* via, uint32_t& next_item,
+                                           uint32_t share = 0u, uint32_t shares = 1u) {
   const uint32_t cap = R.capacity;
   const uint32_t total = S.total;
-  if (!staged && !relist && threadIdx.x == 0) atomicAdd(&B.ctl[g.rep].stage_global, 1u);
+  if (!staged && !relist && threadIdx.x == 0 && share == 0u) atomicAdd(&B.ctl[g.rep].stage_global, 1u);
   const uint32_t nh = home_cells(g);
   const uint32_t H = S.hoff[nh];
-  for (uint32_t h = threadIdx.x; h < H; h += L::kThreads) {
+  for (uint32_t h = share * L::kThreads + threadIdx.x; h < H; h += shares * L::kThreads) {
     const Home a = home_atom(g, S, h);
     const uint32_t i = a.slot;
     double xi, yi, zi;
@@ -1404,7 +1406,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
     return;
   }
   if constexpr (L::kSparse) {
-    build_lanes(B, R, S, g, staged, X, Y, Z, via);
+    build_lanes(B, R, S, g, staged, X, Y, Z, via, share, shares);
     return;
   }
   // Work items: the atoms of each home cell cut into pieces of at most
@@ -1415,8 +1417,9 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
   const uint32_t hv = lane < nh ? S.hoff[lane] : H;
   const uint32_t hn = lane < nh ? S.hoff[lane + 1u] - hv : 0u;
   // a brick of few atoms is cut finer, so that each of its waves has an item
-  const uint32_t each = (H + (uint32_t)(L::kThreads / 64) - 1u) / (uint32_t)(L::kThreads / 64);
-  const uint32_t piece = each < 4u ? 4u : (each < kPiece ? each : kPiece);
+  const uint32_t waves = shares * (uint32_t)(L::kThreads / 64);
+  const uint32_t each = (H + waves - 1u) / waves;
+  const uint32_t piece = each < kLeast ? kLeast : (each < kPiece ? each : kPiece);
   const uint32_t pieces = (hn + piece - 1u) / piece;
   const uint32_t pincl = wave_incl_scan_u32(pieces);
   const uint32_t pv = pincl - pieces;  // lanes past the home cells: the item count
@@ -1424,7 +1427,7 @@ __device__ __forceinline__ void build_part(const Buffers& B, const Replica& R, c
   for (;;) {
     uint32_t item = 0u;
     if (lane == 0u) item = atomicAdd(&next_item, 1u);
-    item = readlane_u32(item, 0);
+    item = readlane_u32(item, 0) * shares + share;
     if (item >= n_items) break;
     const uint32_t hc = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(pv <= item)) - 1u;
     const uint32_t h0 = readlane_u32(hv, hc), n = readlane_u32(hn, hc);
@@ -1557,7 +1560,7 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
     // global memory; either way the overflow is counted.
     const bool over = !staged && home_cells(g) > 1u;
     const bool cut = over && B.parts_on;
-    if (threadIdx.x == 0) {  // mark the brick and record its parts for the PARTS launches
+    if (threadIdx.x == 0 && blockIdx.y == 0u) {  // mark the brick and record its parts for the PARTS launches
       const uint32_t was = B.cut[gb];
       const uint32_t np = cut ? cut_brick(g, S, B.parts + (size_t)gb * kHomeCells) : 0u;
       B.cut[gb] = np;
@@ -1568,7 +1571,7 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
       if (over && !relist) atomicAdd(&B.ctl[g.rep].stage_overflow, 1u);
     }
     if (cut) return;
-    build_part(B, R, S, g, staged, relist != 0, X, Y, Z, via, next_item);
+    build_part(B, R, S, g, staged, relist != 0, X, Y, Z, via, next_item, blockIdx.y, gridDim.y);
   } else {
     each_cut_part<L>(B, [&](uint32_t gb, uint32_t code) {
       const Brick brick = B.bricks[gb];
@@ -3361,6 +3364,23 @@ static void join_side(hipStream_t s, hipStream_t ss, const Side* side, hipError_
   if (e == hipSuccess) e = hipStreamWaitEvent(s, side->join, 0);
 }
 
+// Workgroups that share each brick of a list build: every one stages the brick
+// and takes its share of the work items. A rebuild lasts as long as one brick,
+// and where the bricks that rebuild together leave CUs idle (a small system; one
+// replica of several, which rebuild on their own steps, every ~8) that is most
+// of it: shares until they fill kBuildDense dense workgroups (two a CU) or
+// kBuildSparse sparse ones (five). us/step, one workgroup a brick / this: eight
+// slabs of 15,600 atoms 158 / 139 (a rebuild's launch 72 / 28), 1000 atoms 17.1 /
+// 16.3; with twice as many workgroups the slabs 143 and a batch of 96 replicas
+// 303 / 317.
+constexpr uint32_t kBuildDense = 512, kBuildSparse = 1280, kBuildShares = 8;
+template <class L>
+inline dim3 build_grid(const Buffers& B) {
+  const uint32_t at_once = std::max(1u, layout_count<L>(B) / std::min(B.n_replicas, 8u));
+  const uint32_t shares = (L::kSparse ? kBuildSparse : kBuildDense) / at_once;
+  return dim3(dealt_grid(layout_count<L>(B)), std::min(std::max(shares, 1u), kBuildShares), 1);
+}
+
 hipError_t launch_rebuild(const Buffers& B, hipStream_t s, const Side* side) {
   if (!B.n_atom_blocks) return hipSuccess;
   if (B.chain) {
@@ -3375,9 +3395,9 @@ hipError_t launch_rebuild(const Buffers& B, hipStream_t s, const Side* side) {
   hipError_t e = hipSuccess;
   const hipStream_t ss = fork_side(B, s, side, e);
   if (layout_count<Dense>(B))
-    hipLaunchKernelGGL((k_build<Dense, false>), brick_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, 0);
+    hipLaunchKernelGGL((k_build<Dense, false>), build_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, 0);
   if (layout_count<Sparse>(B))
-    hipLaunchKernelGGL((k_build<Sparse, false>), brick_grid<Sparse>(B), dim3(Sparse::kThreads), 0, ss, B, 0);
+    hipLaunchKernelGGL((k_build<Sparse, false>), build_grid<Sparse>(B), dim3(Sparse::kThreads), 0, ss, B, 0);
   join_side(s, ss, side, e);
   if (B.parts_on && layout_count<Dense>(B)) hipLaunchKernelGGL((k_build<Dense, true>), parts_grid(B), dim3(Dense::kThreads), 0, s, B, 0);
   if (B.parts_on && layout_count<Sparse>(B)) hipLaunchKernelGGL((k_build<Sparse, true>), parts_grid(B), dim3(Sparse::kThreads), 0, s, B, 0);
