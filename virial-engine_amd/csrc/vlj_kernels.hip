@@ -78,6 +78,9 @@ __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, uint32_t l) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
 }
 
+// No instruction is moved across this line by the compiler.
+__device__ __forceinline__ void side_by_side() { __builtin_amdgcn_sched_barrier(0); }
+
 // Reads a word another workgroup wrote, past this CU's L1.
 __device__ __forceinline__ uint32_t load_agent(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1323,7 +1326,13 @@ static_assert(kListStride == 64, "entry pos of a list lies (pos / 8) KB + 2 (pos
 // cells along x, one range of staged atoms. A dilute cell holds a few atoms,
 // so the 64 candidates of a chunk (below) would be mostly empty lanes and
 // every home atom would cost a pass over its chunks; here every lane tests
-// only its own candidates. The lists are the same, entry for entry.
+// only its own candidates. The lists are the same, entry for entry. The bounds of
+// the nine runs and kAhead candidates are read from LDS together: read one by one
+// each waited ~130 cycles (4093 atoms at density 0.1, us per 100 steps and a read
+// of the particles: 2245 one by one, 2157 / 2153 / 2143 with 2 / 4 / 8; a batch of 96
+// replicas, many of them dilute: 15,225 / 15,200 / 15,195 / 15,370).
+constexpr uint32_t kAhead = 4u;
+
 template <class L>
 __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
                                             bool staged, const double* X, const double* Y, const double* Z,
@@ -1337,21 +1346,46 @@ __device__ __forceinline__ void build_lanes(const Buffers& B, const Replica& R, 
     const uint32_t li = a.slot - R.atom_off;
     char* lst = (char*)(B.nbr + list_base(R, li));
     uint32_t found = 0u;
+    auto test = [&](uint32_t q, double xj, double yj, double zj) {
+      const double d2 = dist2(xj - xi, yj - yi, zj - zi);
+      if (d2 < R.list_r2 && q != a.e) {
+        // byte offset (pos / 8) KB + 2 (pos % 8) = 2 pos + 1008 (pos / 8)
+        if (found < cap)
+          *(uint16_t*)(lst + (size_t)(__umul24(found >> 3, 1008u) + 2u * found)) = (uint16_t)list_entry_of(q, staged);
+        found++;
+      }
+    };
+    uint32_t s0[9], s1[9];
+#pragma unroll
     for (uint32_t r = 0; r < 9u; r++) {
       const uint32_t sc = staged_cell(g, a.hz + r / 3u, a.hy + r % 3u, a.hx);
-      const uint32_t s1 = S.off[sc + 3u];
-      for (uint32_t q = S.off[sc]; q < s1; q++) {
-        double xj, yj, zj;
-        staged_pos(R, S, staged, q, X, Y, Z, xj, yj, zj, via);
-        const double d2 = dist2(xj - xi, yj - yi, zj - zi);
-        if (d2 < R.list_r2 && q != a.e) {
-          // byte offset (pos / 8) KB + 2 (pos % 8) = 2 pos + 1008 (pos / 8)
-          if (found < cap)
-            *(uint16_t*)(lst + (size_t)(__umul24(found >> 3, 1008u) + 2u * found)) =
-                (uint16_t)list_entry_of(q, staged);
-          found++;
+      s0[r] = S.off[sc];
+      s1[r] = S.off[sc + 3u];
+    }
+    if (staged) {
+#pragma unroll
+      for (uint32_t r = 0; r < 9u; r++)
+        for (uint32_t q = s0[r]; q < s1[r]; q += kAhead) {
+          double x[kAhead], y[kAhead], z[kAhead];
+#pragma unroll
+          for (uint32_t j = 0; j < kAhead; j++) {
+            const uint32_t e = q + j < s1[r] ? q + j : L::kListPad;  // past the run: the far sentinel
+            x[j] = S.x[e];
+            y[j] = S.y[e];
+            z[j] = S.z[e];
+          }
+          side_by_side();
+#pragma unroll
+          for (uint32_t j = 0; j < kAhead; j++) test(q + j, x[j], y[j], z[j]);
         }
-      }
+    } else {
+#pragma unroll
+      for (uint32_t r = 0; r < 9u; r++)
+        for (uint32_t q = s0[r]; q < s1[r]; q++) {
+          double xj, yj, zj;
+          staged_pos(R, S, false, q, X, Y, Z, xj, yj, zj, via);
+          test(q, xj, yj, zj);
+        }
     }
     // past the capacity the list keeps its first `cap` entries and the
     // overflow is reported (lennard_jones.wgsl:494-497); the last octet is
@@ -1728,9 +1762,6 @@ __device__ __forceinline__ void pair_accumulate(const Replica& R, double dx, dou
 // (FCC-1M 192 us/step either way), which stays.
 constexpr int kPairs = 2;
 static_assert(8 % kPairs == 0, "an octet is whole groups");
-
-// No instruction is moved across this line by the compiler.
-__device__ __forceinline__ void side_by_side() { __builtin_amdgcn_sched_barrier(0); }
 
 template <bool SF>
 __device__ __forceinline__ void pairs_factor(const Replica& R, const double* dx, const double* dy, const double* dz,
@@ -3370,7 +3401,7 @@ static void join_side(hipStream_t s, hipStream_t ss, const Side* side, hipError_
 // replica of several, which rebuild on their own steps, every ~8) that is most
 // of it: shares until they fill kBuildDense dense workgroups (two a CU) or
 // kBuildSparse sparse ones (five). us/step, one workgroup a brick / this: eight
-// slabs of 15,600 atoms 158 / 139 (a rebuild's launch 72 / 28), 1000 atoms 17.1 /
+// slabs of 15,600 atoms 158 / 139 (a rebuild's launch 72 / 38), 1000 atoms 17.1 /
 // 16.3; with twice as many workgroups the slabs 143 and a batch of 96 replicas
 // 303 / 317.
 constexpr uint32_t kBuildDense = 512, kBuildSparse = 1280, kBuildShares = 8;
