@@ -119,3 +119,29 @@ def test_heat_exchange_of_any_size_is_bit_exact(oracle, lj, n):
         rp, rv = ref.read_particles()
         np.testing.assert_array_equal(a["pos"], rp)
         np.testing.assert_array_equal(a["vel"], rv)
+
+
+@pytest.mark.parametrize("n,box,cutoff,shifted", [
+    (343, 8.6, 2.5, True),     # one block of home atoms a brick
+    (344, 11.0, 2.5, False),   # ... and an atom with no neighbour
+    (729, 15.0, 4.5, True),    # a droplet: one to three blocks a brick, lists of up to ~40 octets
+    (1728, 15.0, 4.5, False),  # 1728 staged atoms: each thread sums its own atom's pairs
+])
+def test_heat_current_by_crews_is_bit_exact(oracle, lj, n, box, cutoff, shifted):
+    edge = round(n ** (1.0 / 3.0))
+    grid = np.resize(np.stack(np.meshgrid(*[np.arange(edge)] * 3, indexing="ij"), -1).reshape(-1, 3), (n, 3))
+    rng = np.random.default_rng(23)
+    pos = np.ascontiguousarray((grid - 0.5 * (edge - 1)) * 1.12 + 0.5 * box + rng.uniform(-0.03, 0.03, (n, 3)))
+    if n == 344:
+        pos[-1] = 0.1
+    vel = np.ascontiguousarray(rng.normal(0.0, 0.7, (n, 3)))
+    sim = lj.LennardJones((pos, vel), lj.Settings([box] * 3, cutoff, 0.002, skin=0.3, shifted_force=shifted))
+    ref = oracle.Sim(pos, vel, [box] * 3, cutoff=cutoff, skin=0.3, dt=0.002, shifted_force=shifted)
+    sim.record_heat_current(6)
+    ref.record_heat_current(6)
+    for steps in (0, 1, 2, 16, 1, 20):
+        sim.run(steps)
+        ref.run(steps)
+        sim.sample_heat_current()
+        ref.sample_heat_current()
+    np.testing.assert_array_equal(sim.read_heat_current_raw(), ref.read_heat_current())
