@@ -42,16 +42,17 @@ constexpr double kTuneFills[] = {0.8, 0.9, 1.0};
 // than kSpreadAtoms home atoms (one wave): with the largest bricks that fit
 // the LDS a small system runs on a handful of the 256 CUs, and a launch lasts
 // as long as one brick (staging 3200 atoms, ~480 home atoms in series per
-// wave). One workgroup per CU is the line: us per step with no spread / 256 /
-// 512 / 1024 bricks: 1000 atoms 35 / 27.5 / 27.5 / 27.5, 50,653 atoms 42 /
-// 38.5 / 45.5 / 57 (past one workgroup per CU the halos staged again cost more than the
-// parallelism gives). Fewer than 64 atoms per brick gains nothing (32: within
-// 2%), 128 keeps half of the small system's gain.
+// wave). One workgroup per CU is the line. us per step with no spread / 256 /
+// 512 / 1024 bricks when it was drawn: 1000 atoms 35 / 27.5 / 27.5 / 27.5, 50,653
+// atoms 42 / 38.5 / 45.5 / 57 (past one workgroup per CU the halos staged again
+// cost more than the parallelism gives); with 256 / 384 / 512 now: 50,653 atoms
+// 35.2 / 40.7 / 50.1, eight slabs of 15,600 139 / 176 / 172. Fewer than 64 atoms per
+// brick gains nothing (32: within 2%), 128 keeps half of the small system's gain.
 constexpr double kSpreadBricks = 256.0;
 constexpr double kSpreadAtoms = 64.0;
 // From this many atoms per brick on the LDS limit alone makes enough bricks (a
-// dense brick holds ~460): held to 487, eight slabs of
-// 15,600 atoms ran 1% slower (12% at 244).
+// dense brick holds ~460): eight slabs of 15,600 atoms held to 487 run as without
+// (139 us per step), to 244 a quarter slower.
 constexpr double kSpreadMost = 384.0;
 constexpr double kNoSpread = 1e300;
 // Bricks planned to own at most this many atoms take crews (k_force_crews):
