@@ -332,7 +332,8 @@ int vlj_fixed_sum_device(const double *values, size_t count, double fixed_scale,
 int vlj_debug_state(vlj_sim *sim, double *pos, double *vel, double *acc, uint32_t *orig);
 /* Cell grid of replica 0 after the last rebuild: cell of each slot,
  * total_cells + 1 starts (relative to the replica's first slot), slots in
- * cell order. */
+ * cell order: by the cell of the position each was built from, ascending in
+ * each cell. */
 int vlj_debug_cells(vlj_sim *sim, uint32_t *cell_of, uint32_t *cell_start, uint32_t *sorted);
 /* Neighbour lists of replica 0: counts[n] and entries[n * capacity], row per
  * slot, relative slot indices. */

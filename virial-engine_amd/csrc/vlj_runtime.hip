@@ -1757,8 +1757,24 @@ int vlj_debug_cells(vlj_sim* sim, uint32_t* cell_of, uint32_t* cell_start, uint3
     cell_start[R.total_cells] = R.count;
   }
   if (sorted && rc == VLJ_OK) {
-    // every rebuild leaves the atoms in cell order (R8)
-    for (uint32_t i = 0; i < R.count; i++) sorted[i] = i;
+    // The slots by the cell of the position each was built from, not by the
+    // device's own tables: a rebuild that left an atom in another cell's range
+    // shows here (the right one gives every slot in turn, R8).
+    std::vector<double> built[3];
+    const double* const from[3] = {B.xb, B.yb, B.zb};
+    for (int k = 0; k < 3 && rc == VLJ_OK; k++) {
+      built[k].assign(R.count, 0.0);
+      if (sim->primed) rc = read_dev(sim, built[k].data(), from[k] + R.atom_off, (size_t)R.count * 8);
+    }
+    std::vector<uint32_t> cell(R.count, 0u);
+    for (uint32_t i = 0; i < R.count && rc == VLJ_OK; i++) {
+      uint32_t c[3];
+      for (int k = 0; k < 3; k++) c[k] = host_cell_axis(built[k][i], R.cell_size[k], R.cells[k]);
+      cell[i] = (c[2] * R.cells[1] + c[1]) * R.cells[0] + c[0];
+      sorted[i] = i;
+    }
+    if (rc == VLJ_OK)
+      std::stable_sort(sorted, sorted + R.count, [&](uint32_t a, uint32_t b) { return cell[a] < cell[b]; });
   }
   return rc;
 }
