@@ -335,6 +335,11 @@ int vlj_debug_state(vlj_sim *sim, double *pos, double *vel, double *acc, uint32_
  * cell order: by the cell of the position each was built from, ascending in
  * each cell. */
 int vlj_debug_cells(vlj_sim *sim, uint32_t *cell_of, uint32_t *cell_start, uint32_t *sorted);
+/* How the handle launches its steps: graphs captured since it was created (a
+ * call that steps captures what is missing behind its own work; later calls of
+ * any length capture none until the brick plan or the form of the step
+ * changes), and whether the dense bricks take the crews' launches. */
+int vlj_debug_launches(const vlj_sim *sim, uint64_t out[2]);
 /* Neighbour lists of replica 0: counts[n] and entries[n * capacity], row per
  * slot, relative slot indices. */
 int vlj_debug_lists(vlj_sim *sim, uint32_t *counts, uint32_t *entries);

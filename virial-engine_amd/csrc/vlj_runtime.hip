@@ -2,7 +2,7 @@
 //
 // The handle owns one HIP stream, every device buffer, a 3-slot pinned
 // read-back ring for measurements and the step sequence captured as
-// hipGraphs (of 1, 2, 4, 8 and 16 steps). It replaces the wgpu-side host
+// hipGraphs (of 16, 4 and 2 steps). It replaces the wgpu-side host
 // of crates/virial-particles/src/lennard_jones.rs:443-1375.
 #include <hip/hip_runtime.h>
 
@@ -22,13 +22,19 @@ using namespace vlj;
 namespace {
 
 constexpr int kRing = 3;         // read-back slots (lennard_jones.rs:320)
-// Steps are captured in graphs of 2^k of them, k below kGraphs, each on its
-// first use: a call for few steps between two samples is one or two launches
-// (a graph launch takes ~10 us on the host and leaves a gap of several us).
-// 3458 atoms, a heat-current sample every second step, us per sample with
-// graphs of 1 and 16 only / these: 75.6 / 65.8; a profile sample every 20 steps,
-// 3377 atoms: 437 / 428.
-constexpr uint32_t kGraphs = 5;
+// Steps are captured in graphs of this many; a step past them is launched
+// directly. us a call, a graph of its own length / direct: 1 step of 1000 atoms
+// 41 / 27, of 50,653 56 / 46; 4 steps 73 / 84 and 140 / 156. Two steps are 46 / 42
+// where the rebuild is one launch (k_chain), so those handles take no graph of
+// two, and 79 / 88 where it is four. Eight as two fours: 137 for 129, 272 for 266.
+// A capture takes the host 0.1 (2 steps) to 0.3 ms (16), so the first call that
+// steps leaves all of a handle's graphs behind its own queued work (capture_all;
+// 0.9 ms in all, 1.3 with graphs of two, of which a small system's five steps
+// hide nothing and 20 steps of 1,048,576 atoms everything). Captured on the first
+// use of each length, later calls waited for them: 20 steps after 5 at 1,048,576
+// atoms 0.256 ms a step, 0.235 now.
+constexpr uint32_t kGraphSteps[] = {16, 4, 2};
+constexpr uint32_t kGraphs = 3;
 // Brick planner. Bricks are planned to stage at most kDefaultFill of the
 // LDS staging limit until the tuner has measured the candidates kTuneFills
 // (kTuneSteps steps each) on the handle's own state; a handle of at least
@@ -127,6 +133,8 @@ struct vlj_sim {
   Ring ring[kRing];
   // captured steps, for each orientation of the position sets
   hipGraphExec_t graphs[2][kGraphs] = {};
+  bool all_captured = false;
+  uint64_t captures = 0;  // graphs captured since the handle was created
   // The drift-ahead form (every replica NVE): a step's force launch also
   // drifts the positions of the next step into the second position set
   // (B.x2); `ahead` says it holds them. Each step that uses them swaps the
@@ -464,6 +472,7 @@ void drop_graphs(vlj_sim* s) {
       g = nullptr;
     }
   }
+  s->all_captured = false;
 }
 
 // Captures `steps` steps from the present state; the handle's host state
@@ -487,6 +496,7 @@ int capture(vlj_sim* s, uint32_t steps, hipGraphExec_t* out) {
   }
   if (e != hipSuccess) return fail(s, VLJ_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
   e = hipGraphInstantiateWithFlags(out, g, 0);
+  s->captures++;
   (void)hipGraphDestroy(g);
   if (e != hipSuccess)
     return fail(s, VLJ_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
@@ -1183,17 +1193,21 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   return VLJ_OK;
 }
 
-// 2^k captured steps for the present orientation of the position sets (the
+uint32_t graph_kinds(const vlj_sim* s) { return s->B.chain ? kGraphs - 1u : kGraphs; }
+
+// The graphs that are missing, for both orientations of the position sets (the
 // drift-ahead form swaps them every step: one set of graphs each way).
-int replay(vlj_sim* s, uint32_t k) {
-  hipGraphExec_t& g = s->graphs[s->orient][k];
-  if (!g) {
-    const int rc = capture(s, 1u << k, &g);
-    if (rc != VLJ_OK) return rc;
+int capture_all(vlj_sim* s) {
+  if (s->all_captured) return VLJ_OK;
+  const int ways = drift_ahead(s) ? 2 : 1;
+  int rc = VLJ_OK;
+  for (int o = 0; o < ways; o++) {
+    for (uint32_t k = 0; k < graph_kinds(s) && rc == VLJ_OK; k++)
+      if (!s->graphs[s->orient][k]) rc = capture(s, kGraphSteps[k], &s->graphs[s->orient][k]);
+    if (ways == 2) flip_positions(s);  // twice: as it was
   }
-  HIP_TRY(s, hipGraphLaunch(g, s->stream));
-  if (k == 0 && drift_ahead(s)) flip_positions(s);  // an even count: the sets end as they began
-  return VLJ_OK;
+  s->all_captured = rc == VLJ_OK;
+  return rc;
 }
 
 int enqueue_steps(vlj_sim* s, uint64_t steps) {
@@ -1218,11 +1232,21 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
     if (rc != VLJ_OK) return rc;
     left--;
   }
-  for (uint32_t k = kGraphs; k-- > 0;)
-    for (; left >= 1ull << k; left -= 1ull << k) {
-      rc = replay(s, k);
+  // An even count each: the position sets end as they began. Only the longest
+  // graph is waited for; where a shorter one is missing the steps go directly.
+  const bool stepped = left > 0;
+  for (uint32_t k = 0; k < graph_kinds(s); k++)
+    for (; left >= kGraphSteps[k]; left -= kGraphSteps[k]) {
+      hipGraphExec_t& g = s->graphs[s->orient][k];
+      if (!g && k > 0) break;
+      if (!g) rc = capture(s, kGraphSteps[k], &g);
       if (rc != VLJ_OK) return rc;
+      HIP_TRY(s, hipGraphLaunch(g, s->stream));
     }
+  for (; left > 0; left--) {
+    rc = enqueue_step(s);
+    if (rc != VLJ_OK) return rc;
+  }
   // what the replayed steps leave: drifted positions in B.x2 after
   // drift-ahead steps, none after the others (which use B.x2 as scratch)
   if (steps > 0) {
@@ -1230,7 +1254,8 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
     s->maxima_clear = !s->ahead;
   }
   s->steps += steps;
-  return check_bricks(s);
+  if (stepped) rc = capture_all(s);
+  return rc == VLJ_OK ? check_bricks(s) : rc;
 }
 
 void decode(const vlj_sim* s, uint32_t r, const long long* slots, const Control& c, uint64_t step,
@@ -1619,7 +1644,7 @@ int vlj_record_heat_current(vlj_sim* sim, uint32_t capacity) {
   HIP_TRY(sim, hipMemcpyAsync((void*)&sim->B.rep[0], &sim->rep[0], sizeof(Replica), hipMemcpyHostToDevice,
                               sim->stream));
   HIP_TRY(sim, hipStreamSynchronize(sim->stream));
-  drop_graphs(sim);  // the graphs hold the old buffer pointers
+  // captured steps stay: none of their kernels touches the series
   return VLJ_OK;
 }
 
@@ -1777,6 +1802,13 @@ int vlj_debug_cells(vlj_sim* sim, uint32_t* cell_of, uint32_t* cell_start, uint3
       std::stable_sort(sorted, sorted + R.count, [&](uint32_t a, uint32_t b) { return cell[a] < cell[b]; });
   }
   return rc;
+}
+
+int vlj_debug_launches(const vlj_sim* sim, uint64_t out[2]) {
+  if (!sim || !out) return VLJ_E_INVALID;
+  out[0] = sim->captures;
+  out[1] = sim->B.crews;
+  return VLJ_OK;
 }
 
 int vlj_debug_lists(vlj_sim* sim, uint32_t* counts, uint32_t* entries) {

@@ -102,7 +102,7 @@ extern "C" {
     fn vlj_fixed_sum_device(values: *const f64, n: usize, fixed_scale: f64, out: *mut i64,
                             stream: *mut c_void) -> c_int;
 }
-// Not bound: vlj_debug_state, vlj_debug_cells, vlj_debug_lists, vlj_debug_grid,
+// Not bound: vlj_debug_state, vlj_debug_cells, vlj_debug_launches, vlj_debug_lists, vlj_debug_grid,
 // vlj_debug_counters, vlj_debug_replica_counters, vlj_debug_params, vlj_debug_plan and
 // vlj_debug_parts (planning overrides),
 // vlj_debug_swizzle (the XCD table mapping), vlj_debug_rcp and vlj_debug_rcp32

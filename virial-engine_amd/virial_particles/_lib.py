@@ -136,6 +136,7 @@ SIGNATURES = {
     "vlj_fixed_sum_device": (C.c_int, [_P, _sz, _d, _P, _P]),
     "vlj_debug_state": (C.c_int, [_P, _dp, _dp, _dp, _up]),
     "vlj_debug_cells": (C.c_int, [_P, _up, _up, _up]),
+    "vlj_debug_launches": (C.c_int, [_P, _u64p]),
     "vlj_debug_lists": (C.c_int, [_P, _up, _up]),
     "vlj_debug_grid": (C.c_int, [_P, _up]),
     "vlj_debug_params": (C.c_int, [_P, _dp]),

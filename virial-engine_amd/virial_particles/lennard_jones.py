@@ -585,6 +585,9 @@ class LennardJones:
     def debug_counters(self) -> dict:
         return _debug_counters(self._h)
 
+    def debug_launches(self) -> dict:
+        return _debug_launches(self._h)
+
     def debug_params(self) -> dict:
         out = np.zeros(6)
         self._c(L.lib().vlj_debug_params(self._h, _dptr(out)))
@@ -647,6 +650,12 @@ def _debug_counters(h) -> dict:
     _check(L.lib().vlj_debug_counters(h, out.ctypes.data_as(C.POINTER(C.c_uint64))), h)
     return {"rebuilds": int(out[0]), "stage_overflow_builds": int(out[1]), "list_overflow": int(out[2]),
             "bricks": int(out[3]), "global_cell_builds": int(out[4]), "sparse_bricks": int(out[5])}
+
+
+def _debug_launches(h) -> dict:
+    out = (C.c_uint64 * 2)()
+    _check(L.lib().vlj_debug_launches(h, out), h)
+    return {"captures": out[0], "crews": bool(out[1])}
 
 
 @_render_methods
@@ -733,6 +742,9 @@ class Batch:
 
     def debug_counters(self) -> dict:
         return _debug_counters(self._h)
+
+    def debug_launches(self) -> dict:
+        return _debug_launches(self._h)
 
     def debug_replica_counters(self, replica: int) -> dict:
         """One replica's list rebuilds, cut brick builds, list overflow and
