@@ -338,7 +338,7 @@ int vlj_debug_cells(vlj_sim *sim, uint32_t *cell_of, uint32_t *cell_start, uint3
 /* How the handle launches its steps: graphs captured since it was created (a
  * call that steps captures what is missing behind its own work; later calls of
  * any length capture none until the brick plan or the form of the step
- * changes), and whether the dense bricks take the crews' launches. */
+ * changes), and whether the pair forces of dense bricks take the crews' launch. */
 int vlj_debug_launches(const vlj_sim *sim, uint64_t out[2]);
 /* Neighbour lists of replica 0: counts[n] and entries[n * capacity], row per
  * slot, relative slot indices. */

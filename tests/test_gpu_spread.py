@@ -165,3 +165,37 @@ def test_shared_list_builds_against_the_oracle(oracle, lj):
         np.testing.assert_array_equal(allp["pos"][off:off + len(parts)], pos)
         np.testing.assert_array_equal(allp["vel"][off:off + len(parts)], vel)
         off += len(parts)
+
+
+@pytest.mark.parametrize("replicas,n,density,crews", [
+    (1, 8000, 0.8442, True),     # fewer dense bricks than CUs
+    (1, 16384, 0.8442, False),   # ... and more, of one system
+    (250, 64, 0.36, False),      # ... and of many that are a few cells each
+    (32, 1000, 0.8442, False),
+])
+def test_crews_only_where_every_dense_brick_has_a_cu(oracle, lj, tmp_path, replicas, n, density, crews):
+    side = (n / density) ** (1.0 / 3.0)
+    specs = [(lj.lattice_array(n, side, 1.0, 5 + k), lj.Settings([side] * 3, 2.5, 0.004, skin=0.3))
+             for k in range(replicas)]
+    sim = lj.LennardJones(*specs[0]) if replicas == 1 else lj.Batch(specs)
+    c = sim.debug_counters()
+    assert (c["bricks"] - c["sparse_bricks"] <= 256) == crews
+    assert sim.debug_launches()["crews"] == crews
+    sim.run(40)
+    path = tmp_path / "state"
+    sim.save(path)
+    back = type(sim).load(path)
+    assert back.debug_launches()["crews"] == crews
+    sim.tune(2)
+    c = sim.debug_counters()
+    assert sim.debug_launches()["crews"] == (c["bricks"] - c["sparse_bricks"] <= 256)
+    sim.run(34)
+    back.run(40)
+    a, b = sim.read_particle_array(), back.read_particle_array()
+    np.testing.assert_array_equal(a["pos"], b["pos"])
+    for k in {0, replicas - 1}:
+        parts, st = specs[k]
+        ref = oracle.Sim(np.ascontiguousarray(parts["pos"]), np.ascontiguousarray(parts["vel"]), [side] * 3, cutoff=2.5,
+                         skin=0.3, dt=0.004)
+        ref.run(80)
+        np.testing.assert_array_equal(a["pos"][k * n:(k + 1) * n], ref.read_particles()[0])

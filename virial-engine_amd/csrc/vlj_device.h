@@ -157,6 +157,7 @@ struct Buffers {
   uint32_t n_atom_blocks, n_scan_blocks, n_sort_blocks, n_bricks, n_replicas, n_dense;
   uint32_t nh_inline;  // no replica has more than kInlineBlocks atom blocks: the kernels that scale find the scale
   uint32_t crews;  // the dense bricks are small: crews of waves share their atoms' pairs
+  uint32_t force_crews;  // ... in the force too: a CU for every dense brick
   // 1: a brick whose neighbourhood outgrows LDS is cut into parts, which the
   // PARTS launches after each brick launch take; 0: no PARTS launches, and
   // such a brick runs whole, its positions read through the cell tables

@@ -2168,7 +2168,7 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
 // 17.2, 3458 with the heat current every second step 65.8 / 57 a sample, a
 // driven 10 x 10 x 40 box 42.7 / 39.4. Bricks of more blocks gain nothing: 50,653
 // atoms (200 a brick, crews of two) 36.9 / 43.6 us/step, so the planner's bricks
-// take crews up to kCrewAtoms atoms.
+// take crews up to kCrewAtoms atoms, where each has a CU (kCrewBricks).
 constexpr uint32_t kCrewWaves = Dense::kThreads / 64;
 constexpr uint32_t kCrewOctet = 512;  // factors of one wave's octet: 8 entries x 64 atoms
 
@@ -3528,7 +3528,7 @@ hipError_t force_launches(const Buffers& B, int k, hipStream_t s, const Side* si
   const dim3 gp = parts_grid(B);
   hipError_t e = hipSuccess;
   const hipStream_t ss = fork_side(B, s, side, e);
-  if (layout_count<Dense>(B) && B.crews)
+  if (layout_count<Dense>(B) && B.force_crews)
     hipLaunchKernelGGL((k_force_crews<PREC, SF>), brick_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, k);
   else if (layout_count<Dense>(B))
     hipLaunchKernelGGL((k_force<Dense, PREC, SF, false>), brick_grid<Dense>(B), dim3(Dense::kThreads), 0, s, B, k);

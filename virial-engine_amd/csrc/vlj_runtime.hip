@@ -64,6 +64,13 @@ constexpr double kNoSpread = 1e300;
 // Bricks planned to own at most this many atoms take crews (k_force_crews):
 // two blocks of a wave, four waves to each.
 constexpr double kCrewAtoms = 128.0;
+// ... the force only in handles of at most one dense brick per CU: the crews'
+// kernels take a CU each (256 VGPRs), and two bricks a CU run faster side by side
+// in the plain one. us/step, crews / plain: 196 bricks (8000 atoms) 19.0 / 20.2, 256
+// (12,000) 22.5 / 23.7; 288 (32 x 1000) 54.3 / 47.2, 363 (25,000) 37.3 / 30.6, 405
+// (16,384) 31.9 / 25.1, 500 (250 x 64) 40.9 / 35.0, 1000 (500 x 64) 55.3 / 43.3. A
+// heat-current sample gains there too: 400 bricks (20,000 atoms) 24.2 / 29.2 us.
+constexpr uint32_t kCrewBricks = 256;
 // Atoms per staged cell from which a layer keeps the dense layout however few
 // its bricks stage: a small brick of a liquid fits the sparse layout's 1024
 // atoms, but that layout's build gives each home atom to one lane, which tests
@@ -669,6 +676,12 @@ double plan_spread(const vlj_sim* s) {
   return atoms > kSpreadMost ? kNoSpread : std::max(kSpreadAtoms, atoms);
 }
 
+// Which dense launches crews take, for the brick table in s->bricks.
+void choose_crews(vlj_sim* s) {
+  s->B.crews = plan_spread(s) <= kCrewAtoms;
+  s->B.force_crews = s->B.crews && s->n_dense <= kCrewBricks;
+}
+
 // The brick table from the replicas' brick shapes: every replica's dense
 // bricks, then every sparse one, each part with its larger bricks (more
 // home cells) first and otherwise in layer, row and column order, so that
@@ -748,7 +761,7 @@ int upload_table(vlj_sim* s) {
   }
   B.n_bricks = (uint32_t)nb;
   B.n_dense = s->n_dense;
-  B.crews = plan_spread(s) <= kCrewAtoms;
+  choose_crews(s);
   HIP_TRY(s, hipMemcpy((void*)B.bricks, s->bricks.data(), nb * sizeof(Brick), hipMemcpyHostToDevice));
   HIP_TRY(s, hipMemset(B.cut, 0, std::max<size_t>(nb, 1) * 4));
   HIP_TRY(s, hipMemset(B.cut_groups, 0, std::max<size_t>(ng, 1) * 4));
@@ -1123,7 +1136,7 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   B.bricks = gb;
   B.n_bricks = (uint32_t)s->bricks.size();
   B.n_dense = s->n_dense;
-  B.crews = plan_spread(s) <= kCrewAtoms;
+  choose_crews(s);
   B.parts_on = g_plan.parts >= 0 ? (uint32_t)g_plan.parts : (any_overflow(s, occs) ? 1u : 0u);
   B.n_atom_blocks = (uint32_t)s->atom_blocks.size();
   B.n_scan_blocks = (uint32_t)s->scan_blocks.size();
@@ -1807,7 +1820,7 @@ int vlj_debug_cells(vlj_sim* sim, uint32_t* cell_of, uint32_t* cell_start, uint3
 int vlj_debug_launches(const vlj_sim* sim, uint64_t out[2]) {
   if (!sim || !out) return VLJ_E_INVALID;
   out[0] = sim->captures;
-  out[1] = sim->B.crews;
+  out[1] = sim->B.force_crews;
   return VLJ_OK;
 }
 
@@ -2735,7 +2748,7 @@ int vlj_load(const char* path, vlj_sim** out) {
   s->bricks = bricks;
   s->n_dense = h.n_dense;
   B.n_dense = h.n_dense;
-  B.crews = plan_spread(s) <= kCrewAtoms;
+  choose_crews(s);
   B.parts_on = std::any_of(a.cut.begin(), a.cut.end(), [](uint32_t np) { return np != 0u; }) ? 1u : 0u;
   s->rep_bricks.assign(R, 0u);
   for (const Brick& g : bricks) s->rep_bricks[g.rep]++;
