@@ -199,3 +199,27 @@ def test_crews_only_where_every_dense_brick_has_a_cu(oracle, lj, tmp_path, repli
                          skin=0.3, dt=0.004)
         ref.run(80)
         np.testing.assert_array_equal(a["pos"][k * n:(k + 1) * n], ref.read_particles()[0])
+
+
+@pytest.mark.parametrize("n,rho,sparse", [
+    (20000, 0.3, False),  # small bricks that stage few atoms of a fluid that is not dilute
+    (45000, 0.2, False),
+    (30011, 0.5, False),
+    (45000, 0.05, True),  # ... and a gas, which the sparse layout is for
+])
+def test_a_spread_fluid_takes_one_layout(oracle, lj, n, rho, sparse):
+    side = (n / rho) ** (1.0 / 3.0)
+    if rho >= 0.3:
+        parts, side = lj.fcc_count_array(n, rho, 1.3, 3)
+    else:
+        parts = lj.random_insertion_array(n, [side] * 3, 0.9, 1.3, 3)
+    sim = lj.LennardJones(parts, lj.Settings([side] * 3, 2.5, 0.004, skin=0.3))
+    ref = oracle.Sim(np.ascontiguousarray(parts["pos"]), np.ascontiguousarray(parts["vel"]), [side] * 3, cutoff=2.5,
+                     skin=0.3, dt=0.004)
+    c = sim.debug_counters()
+    assert c["sparse_bricks"] == (c["bricks"] if sparse else 0)
+    for steps in (1, 25):
+        sim.run(steps)
+        ref.run(steps)
+        assert list(sim.measure_now().raw) == list(ref.measure().raw)
+        np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])

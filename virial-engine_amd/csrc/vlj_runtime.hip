@@ -61,6 +61,17 @@ constexpr double kSpreadAtoms = 64.0;
 // (139 us per step), to 244 a quarter slower.
 constexpr double kSpreadMost = 384.0;
 constexpr double kNoSpread = 1e300;
+// The layouts of a spread handle. Its small bricks stage few atoms whatever the
+// fluid, so by their own counts a fluid of 0.15 to 0.5 took both layouts, layer by
+// layer, and the second launch, its fork and its 128 threads for up to 384 home
+// atoms cost 15 to 25 us/step. Past kSpreadAtoms a brick (16,384 atoms) a layer goes
+// by what it would stage without the spread: us/step by the small bricks' counts /
+// by this / with no spread at all: 20,000 atoms at 0.3 52.9 / 24.3 / 38.8, 45,000 at
+// 0.2 56.1 / 27.2 / 33.1. Smaller handles keep their counts' layouts, one launch
+// after the other on one stream (6000 at 0.3 forked 41.9, so 31.7, no spread 38.8)
+// unless more than kSerialReplicas make a rebuild part of every step (12,000 atoms
+// in 21 replicas forked 73.4, so 69.1; 16,000 in 28 71.8 and 74.9).
+constexpr size_t kSerialReplicas = 24;
 // Bricks planned to own at most this many atoms take crews (k_force_crews):
 // two blocks of a wave, four waves to each.
 constexpr double kCrewAtoms = 128.0;
@@ -523,10 +534,16 @@ int capture(vlj_sim* s, uint32_t steps, hipGraphExec_t* out) {
 // the device. A layer whose bricks are held to at most `sparse_fill` of the
 // sparse layout's 1024 atoms takes that layout. A brick of more than one cell
 // owns at most `spread` atoms, by the larger of the replica's and its staged
-// layers' mean occupancy.
+// layers' mean occupancy; from kSpreadAtoms on that only makes bricks smaller, and
+// a layer takes the sparse layout if its bricks would without it too.
 void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fill, double sparse_fill, double spread,
                    std::vector<uint32_t>& bx, std::vector<uint32_t>& by, std::vector<uint8_t>& bz,
                    std::vector<uint8_t>& sparse) {
+  std::vector<uint8_t> dilute;  // layers that take the sparse layout without the spread
+  if (spread > kSpreadAtoms && spread < kNoSpread) {
+    choose_bricks(R, occ, fill, sparse_fill, kNoSpread, bx, by, bz, sparse);
+    dilute = sparse;
+  }
   const int nx = (int)R.cells[0], ny = (int)R.cells[1], nz = (int)R.cells[2];
   const double limit = fill * kStageMax;
   const double sparse_limit = sparse_fill * Sparse::kStageMax;
@@ -627,6 +644,8 @@ void choose_bricks(const Replica& R, const std::vector<uint32_t>& occ, double fi
   // layers' counts, and no more than twice the sparse limit by the
   // replica's mean
   auto sparse_of = [&](const Shape& b, int z, int k) {
+    for (int i = 0; i < k && !dilute.empty(); i++)
+      if (!dilute[z + i]) return 0;
     return b.fits && b.local <= sparse_limit && b.worst <= 2.0 * sparse_limit &&
                    (g_plan.sparse_fill != 0.0 || layers_mean(z, k) < kSparseCell)
                ? 1
@@ -728,6 +747,8 @@ int prime_if_needed(vlj_sim* s) {
 // The side stream for the sparse-layout launches, once both layouts have
 // bricks (default priority).
 int ensure_side(vlj_sim* s) {
+  // a fork costs a small system more than it hides
+  if (plan_spread(s) <= kSpreadAtoms && s->rep.size() <= kSerialReplicas) return VLJ_OK;
   if (s->side.stream || s->n_dense == 0 || s->n_dense == s->bricks.size()) return VLJ_OK;
   HIP_TRY(s, hipStreamCreateWithFlags(&s->side.stream, hipStreamNonBlocking));
   HIP_TRY(s, hipEventCreateWithFlags(&s->side.fork, hipEventDisableTiming));
@@ -1078,14 +1099,10 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
     delete s;
     return fail(nullptr, VLJ_E_HIP, "hipStreamCreate failed");
   }
-  if (s->n_dense > 0 && s->n_dense < s->bricks.size()) {  // both layouts: a side stream (default priority)
-    if (hipStreamCreateWithFlags(&s->side.stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&s->side.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s->side.join, hipEventDisableTiming) != hipSuccess) {
-      free_all(s);
-      delete s;
-      return fail(nullptr, VLJ_E_HIP, "hipStreamCreate failed");
-    }
+  if (ensure_side(s) != VLJ_OK) {
+    free_all(s);
+    delete s;
+    return fail(nullptr, VLJ_E_HIP, "hipStreamCreate failed");
   }
   Buffers& B = s->B;
   const size_t N = s->n_total, C = s->cells_total;
