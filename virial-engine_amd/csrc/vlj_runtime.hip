@@ -2,7 +2,7 @@
 //
 // The handle owns one HIP stream, every device buffer, a 3-slot pinned
 // read-back ring for measurements and the step sequence captured as
-// hipGraphs (of 16, 4 and 2 steps). It replaces the wgpu-side host
+// hipGraphs (of 16 steps and fewer). It replaces the wgpu-side host
 // of crates/virial-particles/src/lennard_jones.rs:443-1375.
 #include <hip/hip_runtime.h>
 
@@ -22,19 +22,22 @@ using namespace vlj;
 namespace {
 
 constexpr int kRing = 3;         // read-back slots (lennard_jones.rs:320)
-// Steps are captured in graphs of this many; a step past them is launched
-// directly. us a call, a graph of its own length / direct: 1 step of 1000 atoms
-// 41 / 27, of 50,653 56 / 46; 4 steps 73 / 84 and 140 / 156. Two steps are 46 / 42
-// where the rebuild is one launch (k_chain), so those handles take no graph of
-// two, and 79 / 88 where it is four. Eight as two fours: 137 for 129, 272 for 266.
+// Steps are captured in graphs of this many; what is left over is launched
+// directly. A launch takes the host ~5 us, a graph ~25 us for its first step and
+// far less for the others, so a step of few launches goes directly and one of many
+// (step_launches) as a graph even alone. us a call, graph of its own length /
+// direct: one step of 3 launches (1000 atoms) 41 / 27, of 7 (Nose-Hoover, 1000) 44 / 39,
+// of 6 (50,653) 56 / 46, of 10 (Nose-Hoover, 20,000) 58 / 66, forked (12 x 2000) 55 to
+// 70 / 91; two steps of 3 launches 46 / 42, of 4 (Langevin, 6000) 55 / 59, of 6 79 / 88,
+// forked 94 / 160; four of 3 73 / 84. Eight as two fours: 137 for 129, 272 for 266.
 // A capture takes the host 0.1 (2 steps) to 0.3 ms (16), so the first call that
 // steps leaves all of a handle's graphs behind its own queued work (capture_all;
-// 0.9 ms in all, 1.3 with graphs of two, of which a small system's five steps
+// 0.9 to 1.3 ms in all, of which a small system's five steps
 // hide nothing and 20 steps of 1,048,576 atoms everything). Captured on the first
 // use of each length, later calls waited for them: 20 steps after 5 at 1,048,576
 // atoms 0.256 ms a step, 0.235 now.
-constexpr uint32_t kGraphSteps[] = {16, 4, 2};
-constexpr uint32_t kGraphs = 3;
+constexpr uint32_t kGraphSteps[] = {16, 4, 2, 1};
+constexpr uint32_t kGraphs = 4;
 // Brick planner. Bricks are planned to stage at most kDefaultFill of the
 // LDS staging limit until the tuner has measured the candidates kTuneFills
 // (kTuneSteps steps each) on the handle's own state; a handle of at least
@@ -79,8 +82,9 @@ constexpr double kCrewAtoms = 128.0;
 // kernels take a CU each (256 VGPRs), and two bricks a CU run faster side by side
 // in the plain one. us/step, crews / plain: 196 bricks (8000 atoms) 19.0 / 20.2, 256
 // (12,000) 22.5 / 23.7; 288 (32 x 1000) 54.3 / 47.2, 363 (25,000) 37.3 / 30.6, 405
-// (16,384) 31.9 / 25.1, 500 (250 x 64) 40.9 / 35.0, 1000 (500 x 64) 55.3 / 43.3. A
-// heat-current sample gains there too: 400 bricks (20,000 atoms) 24.2 / 29.2 us.
+// (16,384) 31.9 / 25.1, 500 (250 x 64) 40.9 / 35.0, 1000 (500 x 64) 55.3 / 43.3 (with
+// FP64 shifted forces 32.7 / 27.0 at 405 and 39.8 / 35.7 at 363, but 34.7 / 35.9 at
+// 400, 20,000 atoms). A heat-current sample gains there too: 400 bricks 24.2 / 29.2.
 constexpr uint32_t kCrewBricks = 256;
 // Atoms per staged cell from which a layer keeps the dense layout however few
 // its bricks stage: a small brick of a liquid fits the sparse layout's 1024
@@ -1223,7 +1227,22 @@ int create(const vlj_particle* all, const uint64_t* offsets, const vlj_settings*
   return VLJ_OK;
 }
 
-uint32_t graph_kinds(const vlj_sim* s) { return s->B.chain ? kGraphs - 1u : kGraphs; }
+// Kernel launches of a step; a fork and join beside another stream count as four.
+uint32_t step_launches(const vlj_sim* s) {
+  uint32_t n = (s->B.chain ? 1u : 4u) + 2u;  // cells to sorted atoms; lists, forces
+  if (s->side.stream) n += 2u + 2u * 4u;
+  if (s->B.parts_on) n += 2u;
+  if (!drift_ahead(s)) n += 1u;
+  if (s->any_nose_hoover) n += 3u;
+  if (s->any_heat_exchange) n += s->B.chain ? 1u : 3u;
+  return n;
+}
+
+// The first lengths of kGraphSteps that the handle replays.
+uint32_t graph_kinds(const vlj_sim* s) {
+  const uint32_t n = step_launches(s);
+  return n < 4u ? 2u : (n < 10u ? 3u : 4u);
+}
 
 // The graphs that are missing, for both orientations of the position sets (the
 // drift-ahead form swaps them every step: one set of graphs each way).
@@ -1262,8 +1281,8 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
     if (rc != VLJ_OK) return rc;
     left--;
   }
-  // An even count each: the position sets end as they began. Only the longest
-  // graph is waited for; where a shorter one is missing the steps go directly.
+  // Only the longest graph is waited for; where a shorter one is missing the
+  // steps go directly.
   const bool stepped = left > 0;
   for (uint32_t k = 0; k < graph_kinds(s); k++)
     for (; left >= kGraphSteps[k]; left -= kGraphSteps[k]) {
@@ -1272,6 +1291,7 @@ int enqueue_steps(vlj_sim* s, uint64_t steps) {
       if (!g) rc = capture(s, kGraphSteps[k], &g);
       if (rc != VLJ_OK) return rc;
       HIP_TRY(s, hipGraphLaunch(g, s->stream));
+      if (kGraphSteps[k] % 2u && drift_ahead(s)) flip_positions(s);
     }
   for (; left > 0; left--) {
     rc = enqueue_step(s);
