@@ -77,6 +77,14 @@ struct Layout {
 };
 using Dense = Layout<kBrickThreads, kStageMax, false>;
 using Sparse = Layout<128, VLJ_SPARSE_STAGE_MAX, true>;
+// Crews (k_force_crews): waves of a dense workgroup, the pair factors of one
+// wave's octet (8 entries x 64 atoms), and the most staged atoms that leave room
+// for every wave's octet, spread over the ends of the three position arrays; 0
+// where a small stage has no such room, and no brick takes crews.
+constexpr uint32_t kCrewWaves = Dense::kThreads / 64;
+constexpr uint32_t kCrewOctet = 512;
+constexpr uint32_t kCrewRoom = (kCrewWaves + 2u) / 3u * kCrewOctet;
+constexpr uint32_t kCrewStaged = Dense::kListPad > kCrewRoom ? Dense::kListPad - kCrewRoom : 0u;
 constexpr int kListStride = 64;   // lists are transposed per block of 64 atoms (one wave)
 constexpr int kSlots = 8;         // fixed-point slots per replica
 constexpr uint32_t kFixedSumBlocks = 256;  // workgroups of the no-allocation fixed-point sum, at most

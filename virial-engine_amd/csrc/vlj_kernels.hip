@@ -2169,13 +2169,6 @@ __global__ void __launch_bounds__(L::kThreads, !PARTS && !L::kSparse ? 4 : 1) k_
 // driven 10 x 10 x 40 box 42.7 / 39.4. Bricks of more blocks gain nothing: 50,653
 // atoms (200 a brick, crews of two) 36.9 / 43.6 us/step, so the planner's bricks
 // take crews up to kCrewAtoms atoms, where each has a CU (kCrewBricks).
-constexpr uint32_t kCrewWaves = Dense::kThreads / 64;
-constexpr uint32_t kCrewOctet = 512;  // factors of one wave's octet: 8 entries x 64 atoms
-
-// The most staged atoms that leave room for every wave's octet, spread over
-// the ends of the three position arrays.
-constexpr uint32_t kCrewStaged = Dense::kListPad - (kCrewWaves + 2u) / 3u * kCrewOctet;
-
 // Where wave w leaves its factors.
 __device__ __forceinline__ double* crew_octet(Stage<Dense>& S, uint32_t w) {
   return S.x + (w % 3u) * (Dense::kStageMax + 64) + (Dense::kListPad - (w / 3u + 1u) * kCrewOctet);

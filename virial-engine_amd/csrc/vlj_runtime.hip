@@ -701,7 +701,7 @@ double plan_spread(const vlj_sim* s) {
 
 // Which dense launches crews take, for the brick table in s->bricks.
 void choose_crews(vlj_sim* s) {
-  s->B.crews = plan_spread(s) <= kCrewAtoms;
+  s->B.crews = kCrewStaged > 0u && plan_spread(s) <= kCrewAtoms;
   s->B.force_crews = s->B.crews && s->n_dense <= kCrewBricks;
 }
 
