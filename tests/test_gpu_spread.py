@@ -223,3 +223,46 @@ def test_a_spread_fluid_takes_one_layout(oracle, lj, n, rho, sparse):
         ref.run(steps)
         assert list(sim.measure_now().raw) == list(ref.measure().raw)
         np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
+
+
+@pytest.mark.parametrize("shifted,precision,thermostat", [(False, 0, 0), (True, 0, 1), (True, 1, 0), (False, 1, 1)])
+def test_crews_beside_cut_bricks(oracle, lj, tmp_path, shifted, precision, thermostat):
+    # a film whose bricks outgrow the stage and are cut, in vapour whose bricks
+    # take crews: planned without limits, loaded from a state file under the rules
+    rng = np.random.default_rng(29)
+    a = 15.0 / 14
+    film = np.stack(np.meshgrid(np.arange(14), np.arange(14), np.arange(11), indexing="ij"), -1).reshape(-1, 3) * a
+    gas = np.stack(np.meshgrid(np.arange(4), np.arange(4), np.arange(6), indexing="ij"), -1).reshape(-1, 3) * 3.6
+    pos = np.concatenate([film + [0.5, 0.5, 12.5], np.where([False, False, True], gas + 26.0, gas + 0.5) % [15.0, 15.0, 36.0]])
+    pos = np.ascontiguousarray((pos + rng.uniform(-0.04, 0.04, pos.shape)) % [15.0, 15.0, 36.0])
+    vel = rng.normal(0.0, 0.8, pos.shape)
+    vel = np.ascontiguousarray(vel - vel.mean(axis=0))
+    box = [15.0, 15.0, 36.0]
+    th = lj.Langevin(0.8, 0.5, 3) if thermostat else None
+    with lj.debug_plan(stage_fill=100.0, sparse_fill=-1.0, parts=True):
+        made = lj.LennardJones((pos, vel), lj.Settings(box, 2.5, 0.003, thermostat=th, skin=0.3, shifted_force=shifted,
+                                                       precision=precision))
+    ref = oracle.Sim(pos, vel, box, cutoff=2.5, skin=0.3, dt=0.003, shifted_force=shifted, precision=precision,
+                     thermostat=thermostat, temperature=0.8 if thermostat else 0.0,
+                     friction=0.5 if thermostat else 0.0, seed=3)
+    made.run(1)
+    ref.run(1)
+    path = tmp_path / "film.state"
+    made.save(path)
+    sim = lj.LennardJones.load(path)
+    assert sim.debug_launches()["crews"] and not made.debug_launches()["crews"]
+    sim.record_heat_current(4)
+    ref.record_heat_current(4)
+    before = sim.debug_counters()
+    for steps in (1, 40, 2, 120):  # fewer than the periodic check of the plan
+        sim.run(steps)
+        ref.run(steps)
+        sim.sample_heat_current()
+        ref.sample_heat_current()
+        assert list(sim.measure_now().raw) == list(ref.measure().raw)
+        np.testing.assert_array_equal(sim.debug_state()[0], ref.state()[0])
+        np.testing.assert_array_equal(sim.debug_state()[1], ref.state()[1])
+    after = sim.debug_counters()
+    cut = after["stage_overflow_builds"] - before["stage_overflow_builds"]
+    assert 0 < cut < (after["rebuilds"] - before["rebuilds"]) * after["bricks"]  # some bricks were cut, not all
+    np.testing.assert_array_equal(sim.read_heat_current_raw(), ref.read_heat_current())
