@@ -129,7 +129,7 @@ struct Control {
   unsigned long long max_moved2;  // FP64 bits; non-negative doubles order as integers
   unsigned long long step;        // steps taken
   uint32_t rebuild;               // this step rebuilds the lists
-  uint32_t reorder;               // ... and moves atoms into cell order
+  uint32_t reorder;               // not used: 0 or 1 in the state files that hold these words
   uint32_t rebuilds;
   uint32_t overflow;
   uint32_t built;

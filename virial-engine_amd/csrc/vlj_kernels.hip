@@ -111,8 +111,7 @@ __device__ void decide_from(const Buffers& B, uint32_t r, double moved2, bool ad
   uint32_t built = c->built;
   uint32_t rebuilds = c->rebuilds;
   bool rebuild = !built || moved2 > R.half_skin2;
-  c->rebuild = rebuild ? 1u : 0u;
-  c->reorder = rebuild ? 1u : 0u;  // R8: every rebuild moves atoms into cell order
+  c->rebuild = rebuild ? 1u : 0u;  // R8: every rebuild moves atoms into cell order
   if (rebuild) {
     c->rebuilds = rebuilds + 1u;
     c->built = 1u;
@@ -243,8 +242,9 @@ __global__ void __launch_bounds__(kBlock) k_drift(Buffers B, int keep_v, int to_
     moved = (unsigned long long)__double_as_longlong(dist2(d[0], d[1], d[2]));
   }
   // One value per workgroup, into one of 64 maxima (lennard_jones.wgsl:215-220
-  // uses one for all: a single address per replica made the step of a 1M-atom
-  // replica 130 us longer).
+  // uses one for all). An atomic of every workgroup on one address per replica --
+  // a ticket, so that the last one could decide -- made the step of a 1M-atom
+  // replica 130 us longer.
   __shared__ unsigned long long wmax[kBlock / 64];
   moved = wave_max_u64(moved);
   if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = moved;
@@ -586,8 +586,9 @@ __global__ void __launch_bounds__(kBlock) k_bin(Buffers B) {
 // that only returns costs ~2.1 us, and four of them (and the reorder's, which
 // the build and the force now do) were a third of a small system's step: 1000
 // atoms 28.0 -> 22.6 us. The limit is what one CU sorts faster than the launches
-// over the whole GPU: 8 us at 1000 atoms, 36 us at 15,600 against their ~30
-// (eight slabs of 15,600 atoms: 113 us a step here, 108 with the launches).
+// over the whole GPU where a replica rebuilds on nearly every step: eight slabs of
+// 15,600 atoms, Nose-Hoover steps without samples, 115.5 us a step here, 105.7 with
+// the launches (a single liquid gains up to there: 12,000 atoms 18.9 for 21.7).
 __global__ void __launch_bounds__(kChainThreads) k_chain(Buffers B) {
   __shared__ uint32_t first[kChainCells + 1];  // counts, then the cell's first place
   __shared__ uint16_t place[kChainAtoms];      // atoms by place, each cell's in any order
@@ -766,7 +767,7 @@ __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
   const Range blk = B.sort_blocks[sb];
   if (!B.ctl[blk.rep].rebuild) return;
   const Replica R = B.rep[blk.rep];
-  __shared__ uint32_t big_c[kBlock], big_start[kBlock], big_n[kBlock];
+  __shared__ uint32_t big_start[kBlock], big_n[kBlock];
   __shared__ uint32_t n_big;
   if (threadIdx.x == 0) n_big = 0u;
   __syncthreads();
@@ -790,7 +791,6 @@ __global__ void __launch_bounds__(kBlock) k_sort(Buffers B) {
       }
     } else {
       const uint32_t k = atomicAdd(&n_big, 1u);
-      big_c[k] = c;
       big_start[k] = start;
       big_n[k] = n;
     }
@@ -903,6 +903,12 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 #define VLJ_READ_PRIO 1
 #endif
 
+// What a crew does while its brick is staged: nothing, where there is none.
+struct NoCrew {
+  __device__ __forceinline__ void cells_known() {}
+  __device__ __forceinline__ void loads_done() {}
+};
+
 // Fills S for brick g from the positions X, Y, Z. Every thread of the
 // workgroup calls it. Returns whether the positions were staged (the
 // neighbourhood holds at most L::kStageMax atoms). `via`, in a rebuild: the
@@ -913,11 +919,6 @@ __device__ __forceinline__ void image_shift(const Replica& R, uint32_t code, dou
 // integer division a cell. us/step before (shuffles, a third scan by one wave,
 // 8 divisions a cell) / with: 1000 atoms 20.1 / 19.2, 50,653 36.9 / 36.0, FCC-1M
 // 196 / 191 (FP32 190 / 184), a batch of 96 replicas 314 / 306.
-struct NoCrew {
-  __device__ __forceinline__ void cells_known() {}
-  __device__ __forceinline__ void loads_done() {}
-};
-
 template <class L, class Crew = NoCrew>
 __device__ bool stage_brick(const Buffers& B, const Replica& R, const Brick& g, const double* X, const double* Y,
                             const double* Z, Stage<L>& S, const uint32_t* via = nullptr, Crew&& crew = Crew()) {
@@ -2019,19 +2020,6 @@ __device__ __forceinline__ PairAcc interactions(const Buffers& B, const Replica&
   return interactions_global<PREC, SF, ENERGIES>(B, R, S, X, Y, Z, i, xi, yi, zi);
 }
 
-// New accelerations, one workgroup per brick (gb: its table entry), and
-// with kick 1 the second half kick v += a dt/2 (v holds the half step).
-// Kick 2, the drift-ahead form (NVE): v holds v(t) and a a(t); the half
-// step v(t) + a(t) dt/2 is formed again exactly as the drift forms it, the
-// kick gives v(t + dt), and the next step's drift follows at once: its half
-// step and x(t + 2 dt) = x(t + dt) + v' dt go to the second position set
-// (x2), which no kernel of this step reads, and the largest moved^2 since
-// the list build into one of the replica's kAheadSlots maxima of the next
-// step (amax_next), so that step needs no drift launch; the set this step's
-// bin read (amax) is zeroed for the step after.
-// `moved`, when the replica's lists were rebuilt on this step: the state in the
-// new order is where the list build left it (positions in xb, the rest in the
-// second set), and goes to the main set from here.
 struct Own {  // an atom's own state before its kick
   double v[3], a[3];
   __device__ __forceinline__ void load(const Buffers& B, uint32_t i, int kick, bool moved) {
@@ -2101,6 +2089,19 @@ __device__ __forceinline__ void finish_brick(const Buffers& B, const Brick& g, u
   }
 }
 
+// New accelerations, one workgroup per brick (gb: its table entry), and
+// with kick 1 the second half kick v += a dt/2 (v holds the half step).
+// Kick 2, the drift-ahead form (NVE): v holds v(t) and a a(t); the half
+// step v(t) + a(t) dt/2 is formed again exactly as the drift forms it, the
+// kick gives v(t + dt), and the next step's drift follows at once: its half
+// step and x(t + 2 dt) = x(t + dt) + v' dt go to the second position set
+// (x2), which no kernel of this step reads, and the largest moved^2 since
+// the list build into one of the replica's kAheadSlots maxima of the next
+// step (amax_next), so that step needs no drift launch; the set this step's
+// bin read (amax) is zeroed for the step after.
+// `moved`, when the replica's lists were rebuilt on this step: the state in the
+// new order is where the list build left it (positions in xb, the rest in the
+// second set), and goes to the main set from here.
 template <int PREC, bool SF, class L>
 __device__ __forceinline__ void force_part(const Buffers& B, const Replica& R, const Stage<L>& S, const Brick& g,
                                            uint32_t gb, bool staged, int kick, bool moved) {
@@ -3235,21 +3236,22 @@ __device__ __forceinline__ void render_part(const Buffers& B, const Replica& R, 
           near += r2 < R.rc2 && r2 < kNearR2 ? 1u : 0u;
         }
       });
-    } else
-    each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
-      const uint32_t e = list_index(entry, staged);
-      double xj, yj, zj;
-      staged_pos(R, S, staged, e, B.x, B.y, B.z, xj, yj, zj);
-      const double r2 = dist2(xj - xi, yj - yi, zj - zi);
-      if (!(r2 < R.rc2)) return;
-      within++;
-      near += r2 < kNearR2 ? 1u : 0u;
-      if (R.drawn == 1u) {
-        const uint32_t c = stage_cell_of(S, e);
-        const uint32_t j = S.base[c] + e;
-        v2 += dist2(B.vx[j], B.vy[j], B.vz[j]);
-      }
-    });
+    } else {
+      each_entry(lst, cnt, [&](uint32_t k, uint32_t entry) {
+        const uint32_t e = list_index(entry, staged);
+        double xj, yj, zj;
+        staged_pos(R, S, staged, e, B.x, B.y, B.z, xj, yj, zj);
+        const double r2 = dist2(xj - xi, yj - yi, zj - zi);
+        if (!(r2 < R.rc2)) return;
+        within++;
+        near += r2 < kNearR2 ? 1u : 0u;
+        if (R.drawn == 1u) {
+          const uint32_t c = stage_cell_of(S, e);
+          const uint32_t j = S.base[c] + e;
+          v2 += dist2(B.vx[j], B.vy[j], B.vz[j]);
+        }
+      });
+    }
     const float w = R.drawn == 1u ? (float)((dist2(v[0], v[1], v[2]) + v2) / (3.0 * (double)(within + 1u)))
                                   : (float)near;
     float4* P = reinterpret_cast<float4*>(B.render_pos);
