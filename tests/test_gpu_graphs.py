@@ -33,17 +33,14 @@ def test_no_call_after_the_first_captures(lj, n, form):
     np.testing.assert_array_equal(sim.debug_state()[1], one.debug_state()[1])
 
 
-def test_no_call_of_a_forked_batch_captures(lj):
-    # both layouts and steps of many launches: single steps are replayed too
-    def batch():
-        specs = []
-        for k in range(4):
-            n, rho = (9000, 0.8442) if k % 2 else (9000, 0.05)
-            side = (n / rho) ** (1.0 / 3.0)
-            parts = lj.lattice_array(n, side, 1.0, 5 + k)
-            specs.append((parts, lj.Settings([side] * 3, 2.5, 0.004, skin=0.3)))
-        return lj.Batch(specs)
-    sim, one = batch(), batch()
+def test_no_call_of_a_forked_batch_captures(oracle, lj):
+    # both layouts on two streams, steps of many launches: single steps are replayed too
+    specs = []
+    for k in range(4):
+        n, rho = (9000, 0.8442) if k % 2 else (9000, 0.05)
+        side = (n / rho) ** (1.0 / 3.0)
+        specs.append((lj.lattice_array(n, side, 1.0, 5 + k), lj.Settings([side] * 3, 2.5, 0.004, skin=0.3)))
+    sim = lj.Batch(specs)
     c = sim.debug_counters()
     assert 0 < c["sparse_bricks"] < c["bricks"]
     sim.run(2)
@@ -51,10 +48,13 @@ def test_no_call_of_a_forked_batch_captures(lj):
     for steps in LENGTHS:
         sim.run(steps)
         assert sim.debug_launches()["captures"] == captured, f"a call of {steps} steps"
-    one.run(2 + sum(LENGTHS))
-    for a, b in zip(sim.measure_now(), one.measure_now()):
-        assert list(a.raw) == list(b.raw)
-    np.testing.assert_array_equal(sim.read_particle_array(), one.read_particle_array())
+    ms, got = sim.measure_now(), sim.read_particle_array()
+    for k, (parts, st) in enumerate(specs):
+        ref = oracle.Sim(np.ascontiguousarray(parts["pos"]), np.ascontiguousarray(parts["vel"]), list(st.box_size),
+                         cutoff=2.5, skin=0.3, dt=0.004)
+        ref.run(2 + sum(LENGTHS))
+        assert list(ms[k].raw) == list(ref.measure().raw), f"replica {k}"
+        np.testing.assert_array_equal(got["pos"][9000 * k:9000 * (k + 1)], ref.read_particles()[0])
 
 
 def test_a_new_plan_or_form_captures_once(lj):
